@@ -555,6 +555,23 @@ def test_mqa_logits_short(num_kv):
     check_mqa(out, q8, k8, ksf, w, ks, ke, stride)
 
 
+@pytest.mark.parametrize("num_q,num_kv", [(1, 447), (1, 448), (9, 449), (8, 897), (3, 2700), (17, 6000), (120, 3100)])
+def test_mqa_logits_key_slices(num_q, num_kv):
+    """Key ranges split over workgroups (slices of 7 or 13 blocks of 64 keys): ranges that end at, before and after
+    a slice's edge, start inside one, and leave gaps between the rows of one workgroup."""
+    print(f"mqa key slices {num_q} x {num_kv}", flush=True)
+    q8, k8, ksf, w = mqa_case(num_q, num_kv, 77 + num_q)
+    rng = np.random.default_rng(num_q)
+    ks = np.zeros(num_q, np.int64)
+    ke = np.full(num_q, num_kv) - np.arange(num_q)[::-1]
+    if num_q > 2:
+        ks[1::3] = num_kv - rng.integers(1, 200, len(ks[1::3]))       # the stream's end only
+        ke[1::3] = num_kv
+        ke[2::3] = rng.integers(0, 200, len(ke[2::3]))                # its start only (a gap between the two)
+    out = run_mqa(q8, k8, ksf, w, ks, ke, (num_kv + 63) // 64 * 64)
+    check_mqa(out, q8, k8, ksf, w, ks, ke, (num_kv + 63) // 64 * 64)
+
+
 def test_mqa_logits_causal_chunk():
     """The benchmark's shape at reduced size: the last 256 rows of one 4096-token sequence, causal."""
     num_q, num_kv, stride = 256, 4096, 4096
