@@ -20,6 +20,10 @@ struct KgFp8Args {
   int m_tiles, n_tiles;
 };
 
+// The deep-ring dense GEMM (kg_fp8_ring.hip) over tiles of bm x bn: one of 32 x 32, 64 x 64, 64 x 128, 128 x 128,
+// 128 x 192.  Sets p.m_tiles and p.n_tiles.
+__attribute__((visibility("hidden"))) int kg_fp8_ring_launch(KgFp8Args& p, int bm, int bn, hipStream_t st);
+
 // Workgroup id -> a contiguous range per XCD (workgroups are dispatched round-robin over the 8 XCDs).
 KG_DEV int kg_xcd_remap(int bid, int total) {
   const int per = total >> 3, rem = total & 7, x = bid & 7, local = bid >> 3;

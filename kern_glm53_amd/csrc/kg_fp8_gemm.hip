@@ -4,7 +4,8 @@
 //   MODE 0  dense:    C[0:m, 0:n] = A . W^T, bf16 out
 //   MODE 1  psum:     per expert g, rows [round_up128(psum[g-1]), psum[g]) with W rows [g n, (g+1) n)
 //   MODE 2  psum + SiLU-mul + per-128 e4m3 requant epilogue (gate columns [0, n/2), up [n/2, n))
-// and a 128 x 128 one-tile-per-workgroup kernel takes dense GEMMs too small for it.
+// and dense GEMMs of fewer tiles go to the deep-ring kernels of kg_fp8_ring.hip or to a 128 x 128 kernel with two
+// workgroups per CU, by the estimate at kg_fp8_gemm.
 //
 // Shared design (CDNA4):
 //   * 256 threads = 4 wave64s in a 2 x 2 grid; a wave owns a quarter of the tile as 32x32 tiles of
@@ -93,8 +94,9 @@ KG_DEV void kg_fp8_epilogue(const KgFp8Args& p, v16f (&acc)[BN / 64][BM / 64], i
   }
 }
 
-// Dense GEMMs too small for the persistent kernel (fewer than 256 tiles of 256 x 256) or whose output
-// strides it cannot store: one 128 x 128 tile per workgroup, K blocks of 128 through two LDS stages.
+// Dense GEMMs of more than one and at most two 128 x 128 tiles per CU: one tile per workgroup, K blocks of 128 through
+// two LDS stages, two workgroups per CU (1700 x 4096 x 6144: 448 tiles in 57.7 us, against 62.1 as two rounds of the
+// deep-ring kernel).
 __global__ __launch_bounds__(256, 2) void kg_fp8_gemm_tile(const KgFp8Args p) {
   constexpr int BM = 128, BN = 128;
   constexpr int TJ = BM / 64;            // m tiles (32 rows) per wave  -> MFMA operand B
@@ -752,16 +754,37 @@ extern "C" int kg_fp8_gemm(const void* a, const void* w, const void* sfa, const 
   p.a = (const u8*)a, p.w = (const u8*)w, p.sfa = (const u32*)sfa, p.sfb = (const u32*)sfb, p.c = (u16*)c;
   p.m = m, p.n = n, p.k = k, p.rows = rows, p.lda = lda, p.ldc = ldc, p.sfa_rows = sfa_rows, p.groups = 1;
   hipStream_t st = (hipStream_t)stream;
-  const long long big = (long long)((m + 255) / 256) * ((n + 255) / 256);
-  // the persistent kernel's epilogue stores 16-byte chunks of 8 columns
-  if (big >= 256 && n % 8 == 0 && ldc % 8 == 0 && kg_aligned(c, 16) && (long long)rows * ldc * 2 < (1ll << 31)) {
-    p.m_tiles = (m + 255) / 256, p.n_tiles = (n + 255) / 256;
-    KG_CHECK(big < (1ll << 31) && (long long)rows * lda < (1ll << 31) && (long long)n * k < (1ll << 31) &&
-             256ll * lda < (1ll << 31));
-    return kg_fp8_launch_persistent<0>(p, big, st);
+  // The kernel and tile shape with the least estimated time: rounds of one tile per slot, each a fixed part and a part
+  // per K block of 128.  The parts are fitted to timings (weights from HBM) of M = 1 .. 4100 at seven N x K from 2752 x
+  // 6144 to 24576 x 6144; over those 130 sizes the pick is within 4% of the best kernel but for one at 12%, and the
+  // deep-ring kernels run 1.56 times as fast as the two others alone (geometric mean).
+  struct Shape {
+    int bm, bn, per_cu;
+    float fixed, block;                          // us
+  };
+  static const Shape shapes[] = {
+      {32, 32, 1, 2.2f, 0.165f},   {64, 64, 1, 2.1f, 0.30f},   {64, 128, 1, 2.2f, 0.40f}, {128, 128, 1, 3.3f, 0.54f},
+      {128, 192, 1, 4.4f, 0.68f},  {128, 128, 2, 4.0f, 1.10f}, {256, 256, 1, 5.0f, 1.36f}};
+  constexpr int TILE = 5, BIG = 6;
+  const int cus = kg_cu_count();
+  // the persistent kernel's epilogue stores 16-byte chunks of 8 columns, and below 256 tiles it is never the best
+  const bool big_ok = (long long)((m + 255) / 256) * ((n + 255) / 256) >= 256 && n % 8 == 0 && ldc % 8 == 0 &&
+                      kg_aligned(c, 16) && (long long)rows * ldc * 2 < (1ll << 31);
+  if (big_ok) KG_CHECK((long long)rows * lda < (1ll << 31));
+  int best = TILE;
+  float best_t = 0.0f;
+  long long tiles = 0;
+  for (int i = 0; i <= (big_ok ? BIG : TILE); ++i) {
+    const Shape& s = shapes[i];
+    const long long t = ((m + s.bm - 1ll) / s.bm) * ((n + s.bn - 1ll) / s.bn), slots = (long long)s.per_cu * cus;
+    const float us = (float)((t + slots - 1) / slots) * (s.fixed + s.block * (float)(k >> 7));
+    if (i == 0 || us < best_t) best = i, best_t = us, tiles = t;
   }
-  p.m_tiles = (m + 127) / 128, p.n_tiles = (n + 127) / 128;
-  return kg_fp8_launch_tile(p, p.m_tiles * p.n_tiles, st);
+  KG_CHECK(tiles < (1ll << 31));
+  p.m_tiles = (m + shapes[best].bm - 1) / shapes[best].bm, p.n_tiles = (n + shapes[best].bn - 1) / shapes[best].bn;
+  if (best == BIG) return kg_fp8_launch_persistent<0>(p, tiles, st);
+  if (best == TILE) return kg_fp8_launch_tile(p, (int)tiles, st);
+  return kg_fp8_ring_launch(p, shapes[best].bm, shapes[best].bn, st);
 }
 
 extern "C" int kg_fp8_gemm_psum(const void* a, const void* w, const void* sfa, const void* sfb, void* c,

@@ -82,6 +82,34 @@ def replay_persistent(M, N, K, rows, lda):
                             check_loads(v, ko, 0, N * K, N * K, f"W tile {mt},{nt} stage {s}")
 
 
+def replay_ring(M, N, K, rows, lda, BM, BN, NW, NS, KBS):
+    """kg_fp8_gemm_ring (kern_glm53_amd/csrc/kg_fp8_ring.hip): one tile per workgroup, NS stages of KBS K blocks, the
+    copies of stage s + NS issued from stage s on (so up to NS stages past the last)."""
+    KS = -(-(K // 128) // KBS)
+    for m0 in range(0, M, BM):
+        m_end = min(M, m0 + BM)
+        for n0 in range(0, N, BN):
+            for s in range(KS + NS):
+                for x in range(KBS):
+                    ko = (s * KBS + x) * 128
+                    for wave in range(NW):
+                        for q in range(BM // 8 // NW):
+                            v = ((q * NW + wave) * 8 + (LANES >> 3)) * lda + chunk(wave & 1)
+                            v = v if ko < K else np.full(64, OOB)
+                            check_loads(v, ko, m0 * lda, (m_end - m0) * lda, rows * lda, f"A {m0},{n0} ko {ko}")
+                        for q in range(BN // 8 // NW):
+                            v = ((q * NW + wave) * 8 + (LANES >> 3)) * K + chunk(wave & 1)
+                            v = v if ko < K else np.full(64, OOB)
+                            check_loads(v, ko, n0 * K, (N - n0) * K, N * K, f"W {m0},{n0} ko {ko}")
+
+
+@pytest.mark.parametrize("BM,BN,NW,NS,KBS", [(32, 32, 4, 8, 2), (64, 64, 4, 8, 1), (64, 128, 4, 4, 1),
+                                             (128, 128, 8, 4, 1), (128, 192, 4, 3, 1)])
+@pytest.mark.parametrize("M,N,K,lda", [(1, 5, 128, 128), (100, 200, 384, 512), (140, 260, 1152, 1152)])
+def test_ring_kernel_dma_in_bounds(BM, BN, NW, NS, KBS, M, N, K, lda):
+    replay_ring(M, N, K, M, lda, BM, BN, NW, NS, KBS)
+
+
 # the dense shapes of tests/test_gpu_gemm.py::test_fp8_gemm (M, N, K, rows, lda) plus single-K-block cases
 SHAPES = [
     (512, 2048, 6144, 512, 6144),

@@ -104,6 +104,36 @@ def test_fp8_gemm(M, N, K, rows, lda, ldc, sfa_rows):
     assert np.all(out[:M, N:] == SENTINEL) and np.all(out[M:] == SENTINEL)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1, 5, 128), (31, 100, 640), (33, 97, 2176),       # 32 x 32 tiles: one K block, odd block counts, past a ring
+    (200, 1201, 384), (193, 1216, 1152),               # 64 x 64
+    (640, 1700, 128), (577, 1729, 1408),               # 64 x 128
+    (1000, 2500, 384), (897, 2433, 640),               # 128 x 128
+    (1500, 3300, 384), (1409, 3265, 1664),             # 128 x 192: fewer K blocks than stages, past a loop body
+    (2000, 3700, 256),                                 # two 128 x 128 workgroups per CU
+])
+def test_fp8_gemm_tile_shapes(M, N, K):
+    """Each tile shape the dense GEMM picks by size, with row, column and K remainders: sampled rows against the
+    oracle and its MFMA model at the bar of test_fp8_gemm, nothing written past m and n."""
+    print(f"fp8 gemm {M}x{N}x{K}", flush=True)
+    ldc = (N + 3) // 4 * 4 + 4
+    a, sfa = quant_act(M, K, M, K, M, seed=M + 5 * N + K)
+    w, sfb = quant_weight(N, K, seed=N + 3 * K)
+    c = filled((M + 2, ldc), SENTINEL, torch.int16)
+    ops.fp8_gemm(d(a), d(w), d(sfa), d(sfb), c, M, n=N, k=K, rows=M, lda=K, ldc=ldc, sfa_rows=M)
+    out = h(c, np.uint16)
+    rs = sample_rows(M, seed=M)
+    R = len(rs)
+    a_s = np.ascontiguousarray(a[rs])
+    sfa_s = np.ascontiguousarray(sfa.reshape(-1, M, 4)[:, rs, :]).reshape(-1)
+    ref32 = ref.fp8_gemm(a_s, w, sfa_s, sfb, R, N, K, K, R)
+    S = ref.fp8_gemm_abs(a_s, w, sfa_s, sfb, R, N, K, K, R)
+    model = ref.fp8_gemm_mfma(a_s, w, sfa_s, sfb, R, N, K, K, R)
+    window = ref.fp8_window_bound(a_s, w, sfa_s, sfb, R, N, K, K, R)
+    check(np.ascontiguousarray(out[rs, :N]), ref32, S, K, f"dense {M}x{N}x{K}", model, window)
+    assert np.all(out[:M, N:] == SENTINEL) and np.all(out[M:] == SENTINEL)
+
+
 @pytest.mark.parametrize("N,K,ldc", [(2624, 6144, 2752), (16384, 2048, 20480), (6144, 16384, 6144)])
 def test_fp8_gemm_bench_shapes_sampled(N, K, ldc):
     """The bench's dense GEMMs at full size (M = 16384: q_a/kv_a, q_b, o_proj): activations quantized on the
