@@ -22,6 +22,7 @@
 //     read as zero and need no clamping.
 #include "kg_device.h"
 #include "kg_host.h"
+#include "kg_ring.h"
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -544,6 +545,171 @@ __global__ __launch_bounds__(256, 1) void kg_gemm_ksplit_kernel(const KgBf16Args
   }
 }
 
+// Wide library GEMMs of few rows (the router of a prompt: 24 to some thousand rows x 256 x 6144).  The ring kernel
+// above has one 128 x 128 tile per 128 rows and column pair: two workgroups at 24 rows, each a chain of 96 stages with
+// B two stages ahead (70 us, of which the MFMA chain is 5).  Here a tile is 32 WM x 32 WN, one 32 x 32 MFMA tile per
+// computing wave, and both operands go through one ring of NS stages of KBS 64-wide K steps with all but one stage in
+// flight; with WM x WN = 1 one wave computes and all four copy.  A stage's fragments are read into one of two register
+// sets while the MFMAs of the stage before run; one barrier per stage, after its first MFMA (this wave's copies of the
+// next stage have landed, its reads of this stage are done), frees this stage's buffer for stage + NS.  The same chain
+// of MFMAs over K per output: sums identical to the kernels above.
+template <bool F32OUT, int WM, int WN, int KBS>
+__global__ __launch_bounds__(256) void kg_gemm_few_kernel(const KgBf16Args p) {
+  constexpr int NW = 4, NS = 8, BM = WM * 32, BN = WN * 32, BLK = (BM + BN) * 128, STAGE = BLK * KBS;
+  constexpr int QA = BM / 8 / NW, QB = BN / 8 / NW, NQ = (QA + QB) * KBS, NT = 4 * KBS;
+  constexpr int FR = 4, CPS = (NQ + NT - 2) / (NT - 1);   // fragments and copies issued after a slot
+  static_assert(BM / 8 % NW == 0 && BN / 8 % NW == 0 && NS * STAGE <= 160 * 1024 && (NS - 1) * NQ < 60, "ring");
+  __shared__ __attribute__((aligned(1024))) u8 st0[STAGE];
+  __shared__ __attribute__((aligned(1024))) u8 st1[STAGE];
+  __shared__ __attribute__((aligned(1024))) u8 st2[STAGE];
+  __shared__ __attribute__((aligned(1024))) u8 st3[STAGE];
+  __shared__ __attribute__((aligned(1024))) u8 st4[STAGE];
+  __shared__ __attribute__((aligned(1024))) u8 st5[STAGE];
+  __shared__ __attribute__((aligned(1024))) u8 st6[STAGE];
+  __shared__ __attribute__((aligned(1024))) u8 st7[STAGE];
+  auto buf = [&](auto i) __attribute__((always_inline)) -> u8* {
+    constexpr int x = decltype(i)::value % NS;
+    if constexpr (x == 0) return st0;
+    else if constexpr (x == 1) return st1;
+    else if constexpr (x == 2) return st2;
+    else if constexpr (x == 3) return st3;
+    else if constexpr (x == 4) return st4;
+    else if constexpr (x == 5) return st5;
+    else if constexpr (x == 6) return st6;
+    else return st7;
+  };
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, wn = wave / WM;
+  const int wid = kg_xcd_remap_b((int)blockIdx.x, (int)gridDim.x);
+  const int mt = wid / p.n_tiles, nt = wid - mt * p.n_tiles;
+  const int m0 = mt * BM, n0 = nt * BN;
+  const int mv = min(BM, p.m - m0), nv = min(BN, p.n - n0);
+  const int KS = ((p.k >> 6) + KBS - 1) / KBS;
+  const __amdgpu_buffer_rsrc_t ra = kg_rsrc_b(p.a + (size_t)m0 * p.a_rs, (long long)(mv - 1) * p.a_rs + 2ll * p.k);
+  const __amdgpu_buffer_rsrc_t rb = kg_rsrc_b(p.b + (size_t)n0 * p.b_rs, (long long)(nv - 1) * p.b_rs + 2ll * p.k);
+
+  // copy instruction q of this wave covers 8 rows from 8 (q NW + wave); NW is even, so a lane's chunk (the swizzled
+  // 128-byte rows of the kernels above) depends on the wave's parity only
+  const int chunk = ((lane & 7) ^ (((wave & 1) << 2) | (lane >> 4))) << 4;
+  unsigned va[QA], vb[QB];
+#pragma unroll
+  for (int q = 0; q < QA; ++q) va[q] = (unsigned)(((q * NW + wave) * 8 + (lane >> 3)) * p.a_rs + chunk);
+#pragma unroll
+  for (int q = 0; q < QB; ++q) vb[q] = (unsigned)(((q * NW + wave) * 8 + (lane >> 3)) * p.b_rs + chunk);
+  auto copy1 = [&](u8* st, int s, int c) __attribute__((always_inline)) {
+    const int x = c / (QA + QB), q = c % (QA + QB), ko = (s * KBS + x) * 128;
+    const bool in = ko < 2 * p.k;                          // a step at or past K reads zeros from past the resource
+    u8* const blk = st + x * BLK + wave * 1024;
+    if (q < QA) kg_ring_copy(ra, blk + q * NW * 1024, in ? va[q] : 0x80000000u, ko);
+    else kg_ring_copy(rb, blk + BM * 128 + (q - QA) * NW * 1024, in ? vb[q - QA] : 0x80000000u, ko);
+  };
+  unsigned offa[4], offb[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const unsigned sw = (unsigned)(((2 * s + (lane >> 5)) ^ (((lane & 31) >> 1) & 7)) << 4);
+    offa[s] = (unsigned)(wm * 32 + (lane & 31)) * 128u + sw;
+    offb[s] = (unsigned)(BM + wn * 32 + (lane & 31)) * 128u + sw;
+  }
+  v16f acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  v8bf fa[2][NT], fb[2][NT];
+  auto frag1 = [&](const u8* st, int set, int f) __attribute__((always_inline)) {
+    const int x = f >> 1;
+    const u8* const b = st + (x >> 2) * BLK;
+    if (f & 1) fa[set][x] = kg_lds_bf16x8(b + offa[x & 3]);
+    else fb[set][x] = kg_lds_bf16x8(b + offb[x & 3]);
+  };
+  auto stage = [&](auto ph, auto comp, int s) __attribute__((always_inline)) {
+    constexpr int PH = decltype(ph)::value;
+    constexpr bool COMP = decltype(comp)::value;
+    u8* const cur = buf(ph);
+    const u8* const nxt = buf(std::integral_constant<int, PH + 1>{});
+    auto slot = [&](auto tt) __attribute__((always_inline)) {
+      constexpr int t = decltype(tt)::value;
+      if constexpr (COMP) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[PH & 1][t], fa[PH & 1][t], acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (t == 0) kg_ring_barrier<(NS - 2) * NQ>();
+      if constexpr (COMP) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int f = t * FR; f < (t + 1) * FR; ++f)
+          if (f < 2 * NT) frag1(nxt, (PH + 1) & 1, f);
+      }
+      if constexpr (t > 0) {
+#pragma unroll
+        for (int c = 0; c < CPS; ++c)
+          if ((t - 1) * CPS + c < NQ) copy1(cur, s + NS, (t - 1) * CPS + c);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    kg_unroll(slot, std::make_integer_sequence<int, NT>{});
+  };
+  auto fill = [&](auto ss) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < NQ; ++c) copy1(buf(ss), decltype(ss)::value, c);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  kg_unroll(fill, std::make_integer_sequence<int, NS>{});
+  kg_ring_barrier<(NS - 1) * NQ>();
+  __builtin_amdgcn_sched_barrier(0);
+  auto run = [&](auto comp) __attribute__((always_inline)) {
+    if constexpr (decltype(comp)::value) {
+#pragma unroll
+      for (int f = 0; f < 2 * NT; ++f) frag1(st0, 0, f);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#define KG_FEW_STAGE(PH)                                        \
+  stage(std::integral_constant<int, (PH)>{}, comp, s + (PH));   \
+  if (s + (PH) + 1 >= KS) break;
+    for (int s = 0;; s += NS) {
+      KG_FEW_STAGE(0)
+      KG_FEW_STAGE(1)
+      KG_FEW_STAGE(2)
+      KG_FEW_STAGE(3)
+      KG_FEW_STAGE(4)
+      KG_FEW_STAGE(5)
+      KG_FEW_STAGE(6)
+      KG_FEW_STAGE(7)
+    }
+#undef KG_FEW_STAGE
+  };
+  // (the waves that only copy run the same barriers in a loop of their own)
+  const bool computes = NW == WM * WN || wave < WM * WN;
+  if constexpr (NW == WM * WN) {
+    run(std::true_type{});
+  } else {
+    if (computes) run(std::true_type{});
+    else run(std::false_type{});
+  }
+  // no copy may still be writing LDS when the workgroup retires
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  const int r = m0 + wm * 32 + (lane & 31);
+  if (!computes || r >= p.m) return;
+  // lane (lane & 31, lane >> 5) holds columns 8 rr + 4 (lane >> 5) .. + 3 of its row (n is a multiple of 8)
+#pragma unroll
+  for (int rr = 0; rr < 4; ++rr) {
+    const int dn = n0 + wn * 32 + rr * 8 + (lane >> 5) * 4;
+    if (dn >= p.n) continue;
+    if constexpr (F32OUT) {
+      *reinterpret_cast<float4*>(p.d + (size_t)r * p.d_rs + 4 * dn) =
+          make_float4(acc[rr * 4 + 0], acc[rr * 4 + 1], acc[rr * 4 + 2], acc[rr * 4 + 3]);
+    } else {
+      uint2 o;
+      o.x = kg_pack_bf16x2(acc[rr * 4 + 0], acc[rr * 4 + 1]);
+      o.y = kg_pack_bf16x2(acc[rr * 4 + 2], acc[rr * 4 + 3]);
+      *reinterpret_cast<uint2*>(p.d + (size_t)r * p.d_rs + 2 * dn) = o;
+    }
+  }
+}
+template __global__ void kg_gemm_few_kernel<true, 1, 1, 2>(const KgBf16Args);
+template __global__ void kg_gemm_few_kernel<true, 2, 2, 1>(const KgBf16Args);
+template __global__ void kg_gemm_few_kernel<false, 1, 1, 2>(const KgBf16Args);
+template __global__ void kg_gemm_few_kernel<false, 2, 2, 1>(const KgBf16Args);
+
 // The library GEMMs take the long-K kernels from this K on (one stage per 64 of K; below it the batched
 // kernel's many-workgroups-per-CU overlap is enough).
 constexpr int KG_LIB_LONG_K = 1024;
@@ -575,12 +741,38 @@ static int kg_gemm_lib_launch(bool f32out, const void* a, const void* b, void* c
     }
     return (int)hipGetLastError();
   }
-  p.m_tiles = (m + 127) / 128, p.n_tiles = (n + 127) / 128;
+  // Tiles of 32 x 32, 64 x 64 or 128 x 128 by the least rounds x time of a tile (us, fixed + per 64 of K; measured with
+  // operands from HBM at K 6144, N 256).  24 rows: 12.3 us against 18.1 and 47.6; 1024: 19.6, 34.6, 71.9; 4096: 72.7,
+  // 37.1, 73.9; 16384: 282, 142, 86.
+  struct Shape {
+    int b;
+    float fixed, step;
+  };
+  static const Shape shapes[] = {{32, 2.0f, 0.18f}, {64, 2.0f, 0.35f}, {128, 3.0f, 0.72f}};
+  constexpr long long CUS = 256;
+  int best = 0;
+  float best_t = 0.0f;
+  for (int i = 0; i < 3; ++i) {
+    const int s = shapes[i].b;
+    const long long t = ((m + s - 1ll) / s) * ((n + s - 1ll) / s);
+    const float us = (float)((t + CUS - 1) / CUS) * (shapes[i].fixed + shapes[i].step * (float)(k >> 6));
+    if (i == 0 || us < best_t) best = i, best_t = us;
+  }
+  const int bt = shapes[best].b;
+  p.m_tiles = (int)((m + bt - 1ll) / bt), p.n_tiles = (int)((n + bt - 1ll) / bt);
   const long long total = (long long)p.m_tiles * p.n_tiles;
   KG_CHECK(total < (1ll << 31));
   const dim3 grid((unsigned)total);
-  if (f32out) hipLaunchKernelGGL((kg_gemm_lib_kernel<true, 128, 128, 1, 2, 7, 3>), grid, dim3(512), 0, st, p);
-  else hipLaunchKernelGGL((kg_gemm_lib_kernel<false, 128, 128, 2, 2, 7, 3>), grid, dim3(256), 0, st, p);
+  if (bt == 32) {
+    if (f32out) hipLaunchKernelGGL((kg_gemm_few_kernel<true, 1, 1, 2>), grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((kg_gemm_few_kernel<false, 1, 1, 2>), grid, dim3(256), 0, st, p);
+  } else if (bt == 64) {
+    if (f32out) hipLaunchKernelGGL((kg_gemm_few_kernel<true, 2, 2, 1>), grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((kg_gemm_few_kernel<false, 2, 2, 1>), grid, dim3(256), 0, st, p);
+  } else {
+    if (f32out) hipLaunchKernelGGL((kg_gemm_lib_kernel<true, 128, 128, 1, 2, 7, 3>), grid, dim3(512), 0, st, p);
+    else hipLaunchKernelGGL((kg_gemm_lib_kernel<false, 128, 128, 2, 2, 7, 3>), grid, dim3(256), 0, st, p);
+  }
   return (int)hipGetLastError();
 }
 

@@ -29,27 +29,7 @@
 #include "kg_host.h"
 
 #include "kg_fp8_common.h"
-
-#include <type_traits>
-#include <utility>
-
-// Waits until at most N of this wave's vector-memory operations and none of its LDS reads are in flight, then for
-// the workgroup.
-template <int N>
-KG_DEV void kg_ring_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-// One copy instruction: 16 bytes a lane from VGPR offset v (range-checked) + ko of resource r to 1 KB of LDS.
-KG_DEV void kg_ring_copy(__amdgpu_buffer_rsrc_t r, u8* dst, unsigned v, int ko) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (KG_LDS void*)dst, 16, v, ko, 0, 0);
-}
-
-// f(0), f(1), ... with the index a compile-time constant.
-template <class F, int... T>
-KG_DEV void kg_unroll(F f, std::integer_sequence<int, T...>) {
-  (f(std::integral_constant<int, T>{}), ...);
-}
+#include "kg_ring.h"
 
 template <int WM, int WN, int TJ, int TI, int NW, int NS, int KBS, int U, int BOFF, int FR, int CPS>
 struct KgRing {

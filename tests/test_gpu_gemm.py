@@ -483,6 +483,28 @@ def test_gemm_long_k_matches_batched(m, n, k, ldc):
     assert np.array_equal(rb, D[:, :n])
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 72, 1024), (33, 264, 1088), (1300, 200, 1088), (2100, 264, 1984)])
+def test_gemm_few_rows_matches_batched(m, n, k):
+    """The wide library GEMMs of few rows, in 32 x 32 and 64 x 64 tiles (by size) with row and column remainders and
+    odd counts of 64-wide K steps: the batched kernel's f32 sums bit for bit, and the bf16 outputs their rounding."""
+    g = synth.generator(11 * m + n)
+    A = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    B = (torch.randn(n, k, generator=g) * 0.02).to(torch.bfloat16).to(DEV)
+    C32 = torch.full((m + 1, n + 8), -7.0, dtype=torch.float32, device=DEV)
+    ops.gemm_f32(A, B, C32, m, n, k, n + 8)
+    C16 = torch.full((m + 1, n + 8), -7.0, dtype=torch.bfloat16, device=DEV)
+    ops.gemm_bf16(A, B, C16, m, n, k, n + 8)
+    R16 = torch.empty(m, 1, n, dtype=torch.bfloat16, device=DEV)
+    ops.bf16_batched(A.view(m, 1, k), B.view(1, n, k), R16, m, n=n, k=k, rows=m, a_strides=(2 * k, 0),
+                     b_strides=(2 * k, 0), d_strides=(2 * n, 0))
+    assert torch.equal(C16[:m, :n], R16[:, 0]) and torch.equal(C32[:m, :n].bfloat16(), R16[:, 0])
+    ref64 = A.double() @ B.double().T
+    S = A.double().abs() @ B.double().abs().T
+    assert bool(((C32[:m, :n] - ref64).abs() <= (k / 16 + 32) * 2.0 ** -24 * S).all())
+    assert bool((C32[:, n:] == -7).all()) and bool((C32[m:] == -7).all())
+    assert bool((C16[:, n:] == -7).all()) and bool((C16[m:] == -7).all())
+
+
 # ------------------------------------------------------------------ MQA logits (a5)
 
 def mqa_case(num_q, num_kv, seed):
