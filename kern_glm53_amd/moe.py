@@ -34,6 +34,11 @@ from . import ops
 
 H, INTER, EXPERTS, TOPK = 6144, 2048, 256, 8     # scripts/gen.py:49-58
 
+# The shared expert's gate_up up to this many tokens: the dense GEMM into bf16 and silu_mul_quant, beyond it the fused
+# grouped GEMM, whose 256 x 256 tiles leave most CUs idle below (24 tokens: 15.2 us against 72.3; 2048: 67.7, 81.7;
+# 2600: 88.1, 82.0).
+SHARED_PAIR_ROWS = 2048
+
 
 def sf_bytes(k: int, rows: int) -> int:
     return ops.sf_words(k) * rows * 4
@@ -75,11 +80,12 @@ class MoEBuffers:
         self.f2 = torch.empty(self.mcap, H, dtype=torch.bfloat16, device=device)
         # the shared expert's gate_up: the fused grouped GEMM over one group owning rows [0, T) (its psum written
         # here, once) needs x_rows in 128-row blocks (it reads A rows up to x_rows rounded up to 128); other
-        # chunks take the dense GEMM into bf16 and silu_mul_quant
+        # chunks, and calls of up to SHARED_PAIR_ROWS tokens, take the dense GEMM into bf16 and silu_mul_quant
         self.fused_shared = x_rows % 128 == 0
         self.spsum = torch.full((1,), T, dtype=torch.int32, device=device)
         self.spsum_T = T                          # the value spsum holds
-        self.sgu = None if self.fused_shared else torch.empty(x_rows, 2 * INTER, dtype=torch.bfloat16, device=device)
+        gu_rows = min(x_rows, SHARED_PAIR_ROWS) if self.fused_shared else x_rows
+        self.sgu = torch.empty(gu_rows, 2 * INTER, dtype=torch.bfloat16, device=device)
         self.sq, self.ssf = u8(x_rows, INTER), u8(sf_bytes(INTER, x_rows))
         self.sh = torch.empty(x_rows, H, dtype=torch.bfloat16, device=device)
 
@@ -112,15 +118,15 @@ def moe_block(xn, xq, xsf, w: MoEWeights, b: MoEBuffers, h, T: int | None = None
     # the shared expert's gate_up (the reference's dense fp8 GEMM into bf16, then silu_mul_quant) as the
     # grouped GEMM with the fused epilogue over one group of T rows: the same codes and scale words (the fused
     # epilogue equals the unfused pair bit for bit), without the [T][4096] bf16 round trip
-    if b.fused_shared:
+    if b.fused_shared and T > SHARED_PAIR_ROWS:
         if T != b.spsum_T:                      # a call of another length than the last one
             b.spsum.fill_(T)
             b.spsum_T = T
         ops.fp8_gemm_psum_silu_quant(xq, w.w_sgu, xsf, w.sf_sgu, b.spsum, b.sq, b.ssf, n=2 * INTER, k=H,
                                      rows=b.x_rows, lda=H, sfa_rows=b.x_rows, sf_rows=b.x_rows, groups=1)
     else:
-        ops.fp8_gemm(xq, w.w_sgu, xsf, w.sf_sgu, b.sgu, T, n=2 * INTER, k=H, rows=b.x_rows, lda=H, ldc=2 * INTER,
-                     sfa_rows=b.x_rows)
+        ops.fp8_gemm(xq, w.w_sgu, xsf, w.sf_sgu, b.sgu, T, n=2 * INTER, k=H, rows=b.sgu.shape[0], lda=H,
+                     ldc=2 * INTER, sfa_rows=b.x_rows)
         ops.silu_mul_quant(b.sgu, INTER, b.sq, b.ssf, b.x_rows, None, T)
     mark("shared_gu_silu_quant")
     ops.fp8_gemm(b.sq, w.w_sdn, b.ssf, w.sf_sdn, b.sh, T, n=H, k=INTER, rows=b.x_rows, lda=INTER, ldc=H,

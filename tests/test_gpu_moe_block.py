@@ -150,3 +150,33 @@ def test_moe_block_against_oracle_chain(T, x_rows):
         moe.moe_block(xn, xq, xsf, Wf, B, out_f)
         torch.cuda.synchronize()
         assert torch.equal(out.view(torch.int16), out_f.view(torch.int16)), sorted(kw)
+
+
+def test_shared_expert_pair_equals_fused(monkeypatch):
+    """The shared expert's two routes (the dense GEMM and silu_mul_quant, or the fused grouped GEMM), on the same tokens:
+    the same codes, scale words and block output, also where a call is shorter than the buffers."""
+    T, t, LIVE = 32, 19, moe.EXPERTS
+    g = synth.generator(77, DEV)
+    xn = torch.randn(128, H, generator=g, device=DEV).bfloat16()
+    xq = torch.empty(128, H, dtype=torch.uint8, device=DEV)
+    xsf = torch.empty(moe.sf_bytes(H, 128), dtype=torch.uint8, device=DEV)
+    ops.quant(xn, H, xq, xsf, 128, H, 128)
+    codes = lambda *s: (torch.randint(0, 0x50, s, generator=g, device=DEV, dtype=torch.int32) |
+                        (torch.randint(0, 2, s, generator=g, device=DEV, dtype=torch.int32) << 7)).to(torch.uint8)
+    sf = lambda groups, n, k: torch.full((groups * moe.sf_bytes(k, n),), 118, dtype=torch.uint8, device=DEV)
+    w13, w2 = codes(1, 2 * INTER, H).expand(LIVE, -1, -1).contiguous(), codes(1, H, INTER).expand(LIVE, -1, -1).contiguous()
+    W = moe.MoEWeights((torch.randn(LIVE, H, generator=g, device=DEV) * 0.01).bfloat16(),
+                       torch.zeros(LIVE, device=DEV), torch.tensor([2.5], dtype=torch.bfloat16, device=DEV),
+                       w13, sf(LIVE, 2 * INTER, H), w2, sf(LIVE, H, INTER), codes(2 * INTER, H), sf(1, 2 * INTER, H),
+                       codes(H, INTER), sf(1, H, INTER))
+    B = moe.MoEBuffers(T, 128, DEV)
+    res = []
+    for limit in (moe.SHARED_PAIR_ROWS, 0):
+        monkeypatch.setattr(moe, "SHARED_PAIR_ROWS", limit)
+        for n in (T, t):
+            out = torch.zeros(T, H, dtype=torch.bfloat16, device=DEV)
+            B.sq.zero_(), B.ssf.zero_()
+            moe.moe_block(xn, xq, xsf, W, B, out, n)
+            res.append((out, B.sq[:n].clone(), B.ssf.view(-1, 128, 4)[:, :n].clone()))
+    for a, b in zip(res[:2], res[2:]):
+        assert all(torch.equal(x.view(torch.uint8), y.view(torch.uint8)) for x, y in zip(a, b))
