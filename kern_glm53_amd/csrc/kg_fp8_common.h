@@ -248,7 +248,7 @@ KG_DEV void kg_fp8_epilogue_silu(const KgFp8Args& p, v16f (&acc)[4][4], u8* stag
     const int lr = arow0 + j * 32;
     const float am = fmaxf(xam[0][lr], xam[1][lr]);
     const u32 e = kg_ue8m0(am, 1e-10f);
-    const float inv = 1.0f / kg_exp2i(e);
+    const float inv = kg_exp2i_inv(e);
     u8* const srow = stage + lr * 128;
 #pragma unroll
     for (int i = 0; i < 2; ++i)

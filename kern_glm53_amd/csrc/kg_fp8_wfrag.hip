@@ -191,7 +191,7 @@ KG_DEV void kg_wf_epilogue_silu(const KgFp8Args& p, v16f (&acc)[4][4], u8* stage
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const float amx = fmaxf(xam[0][sr], xam[1][sr]);
     const u32 e = kg_ue8m0(amx, 1e-10f);
-    const float inv = 1.0f / kg_exp2i(e);
+    const float inv = kg_exp2i_inv(e);
     u8* const srow = stage + sr * 128;
 #pragma unroll
     for (int i = 0; i < 2; ++i)

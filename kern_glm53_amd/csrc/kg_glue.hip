@@ -12,9 +12,8 @@
 // Restates glm_quant / quant4 (source/glm_glue.cu:85-92, 164-175) with 16 lanes x 8 instead of 32 x 4.
 __global__ __launch_bounds__(256) void kg_quant_kernel(const u16* __restrict__ x, int ldx, u8* __restrict__ q,
                                                        u8* __restrict__ sf, int sf_rows, int K, int T) {
-  const long long g = ((long long)blockIdx.x * 256 + threadIdx.x) >> 4;
-  const int nb = K >> 7;
-  if (g >= (long long)T * nb) return;                  // whole 16-lane groups exit together
+  const u32 g = blockIdx.x * 16u + (threadIdx.x >> 4), nb = (u32)K >> 7;
+  if (g >= (u32)T * nb) return;                        // whole 16-lane groups exit together
   const int r = (int)(g / nb), kb = (int)(g % nb), l = threadIdx.x & 15;
   const uint4 raw = *reinterpret_cast<const uint4*>(x + (size_t)r * ldx + kb * 128 + l * 8);
   const u32 w[4] = {raw.x, raw.y, raw.z, raw.w};
@@ -26,7 +25,7 @@ __global__ __launch_bounds__(256) void kg_quant_kernel(const u16* __restrict__ x
   for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
   amax = kg_group_max<16>(amax);
   const u32 e = kg_ue8m0(amax, 1e-10f);
-  const float inv = 1.0f / kg_exp2i(e);
+  const float inv = kg_exp2i_inv(e);
   uint2 o;
   o.x = kg_e4m3x4(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
   o.y = kg_e4m3x4(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
@@ -39,8 +38,8 @@ extern "C" int kg_quant(const void* x, int ldx, void* q, void* sf, int sf_rows, 
   KG_CHECK(kg_aligned(x, 16) && kg_aligned(q, 8));
   if (T == 0) return 0;
   const long long groups = (long long)T * (K / 128);
+  KG_CHECK(groups < 0xfffffff0ll);                     // the kernels index them in 32 bits
   const long long blocks = (groups * 16 + 255) / 256;
-  KG_CHECK(blocks < (1ll << 31));
   hipLaunchKernelGGL(kg_quant_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
                      (const u16*)x, ldx, (u8*)q, (u8*)sf, sf_rows, K, T);
   return (int)hipGetLastError();
@@ -53,9 +52,8 @@ extern "C" int kg_quant(const void* x, int ldx, void* q, void* sf, int sf_rows, 
 __global__ __launch_bounds__(256) void kg_silu_mul_quant_kernel(const u16* __restrict__ gu, int I, u8* __restrict__ q,
                                                                 u8* __restrict__ sf, int sf_rows,
                                                                 const int* __restrict__ n, int rows) {
-  const long long g = ((long long)blockIdx.x * 256 + threadIdx.x) >> 4;
-  const int nb = I >> 7;
-  if (g >= (long long)rows * nb) return;
+  const u32 g = blockIdx.x * 16u + (threadIdx.x >> 4), nb = (u32)I >> 7;
+  if (g >= (u32)rows * nb) return;
   const int r = (int)(g / nb), kb = (int)(g % nb), l = threadIdx.x & 15;
   if (n && r >= *n) return;
   const u16* row = gu + (size_t)r * 2 * I + kb * 128 + l * 8;
@@ -73,7 +71,7 @@ __global__ __launch_bounds__(256) void kg_silu_mul_quant_kernel(const u16* __res
   for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
   amax = kg_group_max<16>(amax);
   const u32 e = kg_ue8m0(amax, 1e-10f);
-  const float inv = 1.0f / kg_exp2i(e);
+  const float inv = kg_exp2i_inv(e);
   uint2 o;
   o.x = kg_e4m3x4(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
   o.y = kg_e4m3x4(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
@@ -87,8 +85,8 @@ extern "C" int kg_silu_mul_quant(const void* gu, int I, void* q, void* sf, int s
   KG_CHECK(kg_aligned(gu, 16) && kg_aligned(q, 8));
   if (rows == 0) return 0;
   const long long groups = (long long)rows * (I / 128);
+  KG_CHECK(groups < 0xfffffff0ll);
   const long long blocks = (groups * 16 + 255) / 256;
-  KG_CHECK(blocks < (1ll << 31));
   hipLaunchKernelGGL(kg_silu_mul_quant_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
                      (const u16*)gu, I, (u8*)q, (u8*)sf, sf_rows, n, rows);
   return (int)hipGetLastError();

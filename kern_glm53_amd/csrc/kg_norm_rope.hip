@@ -46,7 +46,14 @@ KG_DEV uint4 kg_pack8(const float* f) {
   o.w = kg_pack_bf16x2(f[6], f[7]);
   return o;
 }
-KG_DEV float kg_rnd(float x) { return kg_bf16_to_f32(kg_f32_to_bf16(x)); }
+// Pairs rounded to bf16 and back: one conversion, a shift and a mask for two values.
+KG_DEV void kg_rnd8(float* f) {
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    const u32 p = kg_pack_bf16x2(f[i], f[i + 1]);
+    f[i] = kg_u2f(p << 16), f[i + 1] = kg_u2f(p & 0xffff0000u);
+  }
+}
 KG_DEV float kg_xor(float v, int o) { return __shfl_xor(v, o, 64); }
 KG_DEV float kg_rsqrt_rn(float x) { return 1.0f / sqrtf(x); }
 
@@ -80,8 +87,8 @@ KG_DEV uint2 kg_quant8_bf16vals(const float* y, float inv) {
   o.y = kg_e4m3x4(y[4] * inv, y[5] * inv, y[6] * inv, y[7] * inv);
   return o;
 }
-// The same for general f32 values (rope outputs, the fp8 cache's non-power-of-two scale): integer
-// round-to-nearest-even with saturation.
+// The same for the values of the caches (the index key, the fp8 latent with its non-power-of-two scale, whose
+// reciprocal can overflow): integer round-to-nearest-even with saturation.
 KG_DEV uint2 kg_quant8_f32vals(const float* y, float inv) {
   uint2 o;
   o.x = kg_e4m3(y[0] * inv) | (kg_e4m3(y[1] * inv) << 8) | (kg_e4m3(y[2] * inv) << 16) | (kg_e4m3(y[3] * inv) << 24);
@@ -149,7 +156,11 @@ __global__ __launch_bounds__(256) void kg_add_rms_quant_kernel(const u16* __rest
     kg_unpack8(rv[i], x);
     kg_unpack8(gv[i], g);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) y[k] = kg_rnd(kg_rnd(x[k] * rr) * g[k]);
+    for (int k = 0; k < 8; ++k) y[k] = x[k] * rr;
+    kg_rnd8(y);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) y[k] = y[k] * g[k];
+    kg_rnd8(y);
     if (normed) *reinterpret_cast<uint4*>(normed + base + i * 128) = kg_pack8(y);
     if (q) {
       float amax = 0.0f;
@@ -157,7 +168,7 @@ __global__ __launch_bounds__(256) void kg_add_rms_quant_kernel(const u16* __rest
       for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
       amax = kg_row16_max(amax);
       const u32 e = kg_ue8m0(amax, 1e-10f);
-      *reinterpret_cast<uint2*>(q + base + i * 128) = kg_quant8_bf16vals(y, 1.0f / kg_exp2i(e));
+      *reinterpret_cast<uint2*>(q + base + i * 128) = kg_quant8_bf16vals(y, kg_exp2i_inv(e));
       words[i >> 2] |= e << (8 * (i & 3));
     }
   }
@@ -244,13 +255,14 @@ __global__ __launch_bounds__(256) void kg_mla_prep_kernel(
     kg_unpack8(qv[j], f);
     kg_unpack8(*reinterpret_cast<const uint4*>(g_q + kb * 128 + 8 * m), g);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) y[k] = kg_rnd(f[k] * rq * g[k]);
+    for (int k = 0; k < 8; ++k) y[k] = f[k] * rq * g[k];
+    kg_rnd8(y);
     float amax = 0.0f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
     amax = kg_row16_max(amax);
     const u32 e = kg_ue8m0(amax, 1e-10f);
-    *reinterpret_cast<uint2*>(qq + (size_t)r * KG_QL + kb * 128 + 8 * m) = kg_quant8_bf16vals(y, 1.0f / kg_exp2i(e));
+    *reinterpret_cast<uint2*>(qq + (size_t)r * KG_QL + kb * 128 + 8 * m) = kg_quant8_bf16vals(y, kg_exp2i_inv(e));
     word |= e << (8 * j);
   }
   if (m == 0) qsf[(size_t)wq * sf_rows + r] = word;
@@ -261,7 +273,8 @@ __global__ __launch_bounds__(256) void kg_mla_prep_kernel(
   float g[8], kn[8];
   kg_unpack8(*reinterpret_cast<const uint4*>(g_kv + 8 * lane), g);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) kn[k] = kg_rnd(kvf[k] * rk * g[k]);
+  for (int k = 0; k < 8; ++k) kn[k] = kvf[k] * rk * g[k];
+  kg_rnd8(kn);
   if constexpr (FP8) {
     // tile wq = columns 128 wq .. : scale amax / 448 (not a power of two), 0 for an all-zero tile
     float amax = 0.0f;
@@ -411,8 +424,12 @@ __global__ __launch_bounds__(256) void kg_q_post_kernel(const u16* __restrict__ 
 #pragma unroll
     for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(f[k]));
     amax = kg_row16_max(amax);
-    const float sc = kg_exp2i(kg_ue8m0(amax, 1e-4f));
-    *reinterpret_cast<uint2*>(iq + ((size_t)r * KG_IH + ih) * KG_ID + 8 * m) = kg_quant8_f32vals(f, 1.0f / sc);
+    const u32 e = kg_ue8m0(amax, 1e-4f);
+    const float sc = kg_exp2i(e), inv = kg_exp2i_inv(e);
+    uint2 o;
+    o.x = kg_e4m3x4_signed(f[0] * inv, f[1] * inv, f[2] * inv, f[3] * inv);
+    o.y = kg_e4m3x4_signed(f[4] * inv, f[5] * inv, f[6] * inv, f[7] * inv);
+    *reinterpret_cast<uint2*>(iq + ((size_t)r * KG_IH + ih) * KG_ID + 8 * m) = o;
     if (m == 0) {
       float w = kg_bf16_to_f32(iw[(size_t)r * KG_IH + ih]);
       w *= sc;

@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void kg_requant_kernel(const u8* __restrict__ 
   const float scale = s[(size_t)blockIdx.x * (K / 128) + blockIdx.y];
   const float amax = fabsf(kg_e4m3_to_f32(cmax) * scale);
   const u32 e = kg_ue8m0(amax, 1e-4f);
-  const float inv = 1.0f / kg_exp2i(e);
+  const float inv = kg_exp2i_inv(e);
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const int r = row0 + 16 * j;

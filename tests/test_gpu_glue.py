@@ -34,6 +34,23 @@ def test_quant_bit_exact(T, K, ldx, sf_rows):
     assert np.array_equal(h(sf, np.uint8), sf_ref)
 
 
+def test_quant_scale_boundaries():
+    """Block amax values at, just below and just above 1.75 * 2^E, at 2^E and at the largest mantissa, for every
+    exponent E from zero and subnormals up to infinity: the scale byte steps exactly there."""
+    mant = np.array([0x00, 0x5f, 0x60, 0x61, 0x7f], np.uint16)
+    x = np.zeros((5, 256, 128), np.uint16)
+    x[:, :, 17] = (np.arange(256, dtype=np.uint16)[None, :] << 7) | mant[:, None]
+    x[:, 255, 17] = 0x7f80
+    x[:, :, 18] = x[:, :, 17] | 0x8000
+    x[:, :, 19] = np.where(x[:, :, 17] >= 0x80, x[:, :, 17] - 0x80, 0)
+    x = x.reshape(5, -1)
+    q_ref, sf_ref = ref.quant(x, 32768, 5, 5)
+    q, sf = filled((5, 32768), 0), filled((ref.sf_words(32768) * 5 * 4,), 0)
+    ops.quant(d(x), 32768, q, sf, 5, 32768, 5)
+    assert np.array_equal(h(sf, np.uint8), sf_ref)
+    assert np.array_equal(h(q, np.uint8)[:, :255 * 128], q_ref[:, :255 * 128])   # (an infinite block has no codes)
+
+
 def test_quant_full_size_properties():
     """16384 x 6144 (the dense GEMMs' activation): every (row, block) satisfies the UE8M0 contract and
     matches the oracle on a sample of rows."""

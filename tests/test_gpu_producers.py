@@ -200,6 +200,24 @@ def test_q_post_bit_exact(T, full, ldb):
     assert np.array_equal(h(wout_d, np.uint32), wout.view(np.uint32))
 
 
+def test_q_post_wide_values():
+    """Indexer queries over 60 powers of two, so that codes of every size, subnormal ones and zeros come up behind one
+    scale, with a NaN of either sign, whose code keeps the sign."""
+    T = 9
+    rng = np.random.default_rng(11)
+    qb = bf16_bits(spread(rng, (T, 20480), -30, 30) * np.exp2(rng.integers(-12, 13, (T, 160)).repeat(128, 1)))
+    qb[:, 16384:].reshape(T, 32, 128)[3, 5, 70:72] = (0x7fc0, 0xffc0)
+    rope, pos = rope_table(80), rng.integers(0, 80, T).astype(np.int32)
+    qmla, iq = np.zeros((T, 64, 576), np.uint16), np.zeros((T, 32, 128), np.uint8)
+    iw, wout = bf16_bits(rng.standard_normal((T, 32))), np.zeros((T, 32), np.float32)
+    qmla_d, iq_d, wout_d = d(qmla), d(iq), d(wout)
+    ref.q_post(qb, rope, pos, qmla, iq, iw, wout, True, T)
+    ops.q_post(d(qb), 20480, d(rope), d(pos), qmla_d, iq_d, d(iw), wout_d, True, T, rope_rows=80)
+    assert np.array_equal(h(qmla_d, np.uint16), qmla)
+    assert np.array_equal(h(iq_d, np.uint8), iq)
+    assert np.array_equal(h(wout_d, np.uint32), wout.view(np.uint32))
+
+
 def test_q_post_full_chunk_sampled():
     T, ldb, rope_rows = 16384, 20480, 65536
     print("q_post full chunk", flush=True)
