@@ -193,7 +193,8 @@ extern "C" int kg_add_rms_quant(const void* a, void* res, const void* gamma, voi
 
 // Lane (wq, m): q_a chunks m of blocks 4 wq + 2 s + i (the reference's warps 2 wq + s, its lanes 2m, 2m + 1);
 // kv_a chunk `lane` (columns 8 lane .. +7: the reference's threads 4 lane .. 4 lane + 3, warp lane >> 3);
-// k_pe chunk `lane` for lanes 0-7; the indexer key's chunk m in lanes 0-15 (the reference's warp 7).
+// k_pe chunk `lane` for lanes 0-7; the indexer key's chunk m in lanes 0-15 (the reference's warp 7).  Two waves a row,
+// q_a in one and the caches' rows in the other: their reductions are independent chains.
 template <bool FP8>
 __global__ __launch_bounds__(256) void kg_mla_prep_kernel(
     const u16* __restrict__ x, int lda, const u16* __restrict__ g_q, const u16* __restrict__ g_kv,
@@ -201,34 +202,61 @@ __global__ __launch_bounds__(256) void kg_mla_prep_kernel(
     u8* __restrict__ kv, u8* __restrict__ idx, const u16* __restrict__ ik_w, const u16* __restrict__ ik_b,
     u8* __restrict__ qq, u32* __restrict__ qsf, int sf_rows, int T, long long num_slots, int rope_rows) {
   const int lane = threadIdx.x & 63, wq = lane >> 4, m = lane & 15;
-  const int r = kg_rows_remap((int)blockIdx.x, (int)gridDim.x) * 4 + (threadIdx.x >> 6);
+  const int unit = __builtin_amdgcn_readfirstlane(kg_rows_remap((int)blockIdx.x, (int)gridDim.x) * 4 +
+                                                  (int)(threadIdx.x >> 6));
+  const int r = unit >> 1;
   if (r >= T) return;
   const u16* row = x + (size_t)r * lda;
-  uint4 qv[4];
+  if ((unit & 1) == 0) {
+    uint4 qv[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) qv[j] = *reinterpret_cast<const uint4*>(row + (4 * wq + j) * 128 + 8 * m);
+    for (int j = 0; j < 4; ++j) qv[j] = *reinterpret_cast<const uint4*>(row + (4 * wq + j) * 128 + 8 * m);
+    // rq: chains [s][e] over blocks i = 0, 1 of warp 2 wq + s
+    float c[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float f[8];
+      kg_unpack8(qv[j], f);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) c[j >> 1][0] = __builtin_fmaf(f[k], f[k], c[j >> 1][0]);
+#pragma unroll
+      for (int k = 4; k < 8; ++k) c[j >> 1][1] = __builtin_fmaf(f[k], f[k], c[j >> 1][1]);
+    }
+    float t0 = kg_warp_sum_pairs(c[0][0], c[0][1]), t1 = kg_warp_sum_pairs(c[1][0], c[1][1]);
+    t0 += kg_xor(t0, 32), t1 += kg_xor(t1, 32);
+    t0 += kg_xor(t0, 16), t1 += kg_xor(t1, 16);
+    const float rq = kg_rsqrt_rn((t0 + t1) / (float)KG_QL + KG_EPS);
+
+    // q_c = bf16(q_a * rq * g_q) quantized per block: blocks 4 wq .. 4 wq + 3 are scale word wq
+    u32 word = 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int kb = 4 * wq + j;
+      float f[8], g[8], y[8];
+      kg_unpack8(qv[j], f);
+      kg_unpack8(*reinterpret_cast<const uint4*>(g_q + kb * 128 + 8 * m), g);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) y[k] = f[k] * rq * g[k];
+      kg_rnd8(y);
+      float amax = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
+      amax = kg_row16_max(amax);
+      const u32 e = kg_ue8m0(amax, 1e-10f);
+      *reinterpret_cast<uint2*>(qq + (size_t)r * KG_QL + kb * 128 + 8 * m) = kg_quant8_bf16vals(y, kg_exp2i_inv(e));
+      word |= e << (8 * j);
+    }
+    if (m == 0) qsf[(size_t)wq * sf_rows + r] = word;
+    return;
+  }
+
+  const long long s = slot[r];
+  const int p = pos[r];
   const uint4 kvv = *reinterpret_cast<const uint4*>(row + KG_QL + 8 * lane);
   uint4 pev = {0u, 0u, 0u, 0u}, wkv = {0u, 0u, 0u, 0u};
   if (lane < 8) pev = *reinterpret_cast<const uint4*>(row + KG_QL + KG_KVL + 8 * lane);
   if (idx && lane < 16) wkv = *reinterpret_cast<const uint4*>(row + KG_QL + KG_KVL + 2 * KG_HALF + 8 * lane);
-  const long long s = slot[r];
-  const int p = pos[r];
-
-  // rq: chains [s][e] over blocks i = 0, 1 of warp 2 wq + s
-  float c[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    float f[8];
-    kg_unpack8(qv[j], f);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) c[j >> 1][0] = __builtin_fmaf(f[k], f[k], c[j >> 1][0]);
-#pragma unroll
-    for (int k = 4; k < 8; ++k) c[j >> 1][1] = __builtin_fmaf(f[k], f[k], c[j >> 1][1]);
-  }
-  float t0 = kg_warp_sum_pairs(c[0][0], c[0][1]), t1 = kg_warp_sum_pairs(c[1][0], c[1][1]);
-  t0 += kg_xor(t0, 32), t1 += kg_xor(t1, 32);
-  t0 += kg_xor(t0, 16), t1 += kg_xor(t1, 16);
-  const float rq = kg_rsqrt_rn((t0 + t1) / (float)KG_QL + KG_EPS);
+  if (s < 0 || s >= num_slots || p < 0 || p >= rope_rows) return;
 
   // rk: reference thread 4 lane + u holds columns 2u, 2u + 1 of this chunk; its warp lane >> 3, its lane
   // 4 (lane & 7) + u, so distances 16, 8, 4 are lanes ^ 4, ^ 2, ^ 1 and distances 2, 1 are u ^ 2, u ^ 1
@@ -246,28 +274,6 @@ __global__ __launch_bounds__(256) void kg_mla_prep_kernel(
   tk += kg_xor(tk, 8);                                    // w ^ 1
   const float rk = kg_rsqrt_rn(tk / (float)KG_KVL + KG_EPS);
 
-  // q_c = bf16(q_a * rq * g_q) quantized per block: blocks 4 wq .. 4 wq + 3 are scale word wq
-  u32 word = 0u;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int kb = 4 * wq + j;
-    float f[8], g[8], y[8];
-    kg_unpack8(qv[j], f);
-    kg_unpack8(*reinterpret_cast<const uint4*>(g_q + kb * 128 + 8 * m), g);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) y[k] = f[k] * rq * g[k];
-    kg_rnd8(y);
-    float amax = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
-    amax = kg_row16_max(amax);
-    const u32 e = kg_ue8m0(amax, 1e-10f);
-    *reinterpret_cast<uint2*>(qq + (size_t)r * KG_QL + kb * 128 + 8 * m) = kg_quant8_bf16vals(y, kg_exp2i_inv(e));
-    word |= e << (8 * j);
-  }
-  if (m == 0) qsf[(size_t)wq * sf_rows + r] = word;
-
-  if (s < 0 || s >= num_slots || p < 0 || p >= rope_rows) return;
   const u16* cs = rope + (size_t)p * 2 * KG_HALF;
   u8* dst = kv + s * (FP8 ? KG_KV8 : KG_MLA * 2);
   float g[8], kn[8];
@@ -344,14 +350,14 @@ static int kg_mla_prep_launch(const void* x, int lda, const void* g_q, const voi
                               const int* pos, const long long* slot, void* kv, void* idx, const void* ik_w,
                               const void* ik_b, void* qq, void* qsf, int sf_rows, int T, long long num_slots,
                               int rope_rows, void* stream) {
-  KG_CHECK(x && g_q && g_kv && rope && pos && slot && kv && qq && qsf && T >= 0 && T <= sf_rows);
+  KG_CHECK(x && g_q && g_kv && rope && pos && slot && kv && qq && qsf && T >= 0 && T <= sf_rows && T < 1 << 30);
   KG_CHECK(lda >= KG_QL + KG_KVL + 2 * KG_HALF + (idx ? KG_ID : 0) && lda % 8 == 0 && num_slots >= 0 &&
            rope_rows >= 0);
   KG_CHECK(!idx || (ik_w && ik_b && kg_aligned(idx, 8) && kg_aligned(ik_w, 16) && kg_aligned(ik_b, 16)));
   KG_CHECK(kg_aligned(x, 16) && kg_aligned(g_q, 16) && kg_aligned(g_kv, 16) && kg_aligned(rope, 8) &&
            kg_aligned(kv, 16) && kg_aligned(qq, 8) && kg_aligned(qsf, 4));
   if (T == 0) return 0;
-  hipLaunchKernelGGL(kg_mla_prep_kernel<FP8>, dim3((T + 3) / 4), dim3(256), 0, (hipStream_t)stream, (const u16*)x,
+  hipLaunchKernelGGL(kg_mla_prep_kernel<FP8>, dim3((T + 1) / 2), dim3(256), 0, (hipStream_t)stream, (const u16*)x,
                      lda, (const u16*)g_q, (const u16*)g_kv, (const u16*)rope, pos, slot, (u8*)kv, (u8*)idx,
                      (const u16*)ik_w, (const u16*)ik_b, (u8*)qq, (u32*)qsf, sf_rows, T, num_slots, rope_rows);
   return (int)hipGetLastError();
@@ -375,48 +381,57 @@ extern "C" int kg_mla_prep_fp8(const void* x, int lda, const void* g_q, const vo
 // ============================================================================ q post
 
 // q_pe: 64 heads x 8 chunks of 4 pairs = 512 chunks, lane takes chunk it * 64 + lane (head it * 8 + lane / 8,
-// pairs 4 (lane & 7) ..).  Indexer query: head it * 4 + wq, chunk m; a 16-lane group per head.
+// pairs 4 (lane & 7) ..).  Indexer query: head it * 4 + wq, chunk m; a 16-lane group per head.  A row is two units
+// of KG_QP_IT steps `it` of the q_pe part and two of the indexer's, a wave each: at 2050 rows a wave per row left two
+// waves on a SIMD, each a chain of loads, arithmetic and stores (the three row kernels 68.2 us; 63.7 with this and the
+// two waves a row of MLA prep).
+constexpr int KG_QP_IT = 4, KG_QP_UNITS = 8 / KG_QP_IT;
 __global__ __launch_bounds__(256) void kg_q_post_kernel(const u16* __restrict__ qb, int ldb, const u16* __restrict__ rope,
                                                         const int* __restrict__ pos, u16* __restrict__ qmla,
                                                         u8* __restrict__ iq, const u16* __restrict__ iw,
                                                         float* __restrict__ wout, int full, int T, int rope_rows) {
   const int lane = threadIdx.x & 63, wq = lane >> 4, m = lane & 15, sub = lane & 7;
-  const int r = kg_rows_remap((int)blockIdx.x, (int)gridDim.x) * 4 + (threadIdx.x >> 6);
+  const int unit = __builtin_amdgcn_readfirstlane(kg_rows_remap((int)blockIdx.x, (int)gridDim.x) * 4 +
+                                                  (int)(threadIdx.x >> 6));
+  const int per = full ? 2 * KG_QP_UNITS : KG_QP_UNITS, r = (int)((unsigned)unit / (unsigned)per), part = unit - r * per;
   if (r >= T) return;
-  const int p = pos[r];
+  const int p = pos[r], it0 = part % KG_QP_UNITS * KG_QP_IT;
   if (p < 0 || p >= rope_rows) return;
   const u16* row = qb + (size_t)r * ldb;
   const u16* cs = rope + (size_t)p * 2 * KG_HALF;
-  float cv[4], sv[4];
+  uint4 v[KG_QP_IT];
+#pragma unroll
+  for (int i = 0; i < KG_QP_IT; ++i) {
+    const int it = it0 + i;
+    v[i] = *reinterpret_cast<const uint4*>(row + (part < KG_QP_UNITS
+                                                      ? (it * 8 + (lane >> 3)) * KG_QHD + KG_NOPE + 8 * sub
+                                                      : KG_HEADS * KG_QHD + (it * 4 + wq) * KG_ID + 8 * m));
+  }
+  float cv[4], sv[4];                            // the indexer's chunks m < 8 take pairs 4m .. 4m + 3
   kg_unpack4(*reinterpret_cast<const uint2*>(cs + 4 * sub), cv);
   kg_unpack4(*reinterpret_cast<const uint2*>(cs + KG_HALF + 4 * sub), sv);
-  uint4 v[8];
+  if (part < KG_QP_UNITS) {
 #pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int h = it * 8 + (lane >> 3);
-    v[it] = *reinterpret_cast<const uint4*>(row + h * KG_QHD + KG_NOPE + 8 * sub);
+    for (int i = 0; i < KG_QP_IT; ++i) {
+      const int h = (it0 + i) * 8 + (lane >> 3);
+      float f[8];
+      kg_unpack8(v[i], f);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) kg_rope(f[2 * u], f[2 * u + 1], cv[u], sv[u]);
+      *reinterpret_cast<uint4*>(qmla + ((size_t)r * KG_HEADS + h) * KG_MLA + KG_KVL + 8 * sub) = kg_pack8(f);
+    }
+    return;
   }
-#pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int h = it * 8 + (lane >> 3);
-    float f[8];
-    kg_unpack8(v[it], f);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) kg_rope(f[2 * u], f[2 * u + 1], cv[u], sv[u]);
-    *reinterpret_cast<uint4*>(qmla + ((size_t)r * KG_HEADS + h) * KG_MLA + KG_KVL + 8 * sub) = kg_pack8(f);
-  }
-  if (!full) return;
   // indexer query: this lane's chunk m of heads it * 4 + wq; rope for chunks 0-7 (pairs 4m ..)
   const bool roped = m < 8;
+  u16 iwv[KG_QP_IT];
 #pragma unroll
-  for (int it = 0; it < 8; ++it) v[it] = *reinterpret_cast<const uint4*>(row + KG_HEADS * KG_QHD + (it * 4 + wq) * KG_ID + 8 * m);
-  kg_unpack4(*reinterpret_cast<const uint2*>(cs + 4 * sub), cv);      // m < 8 reads pairs 4m .. 4m + 3
-  kg_unpack4(*reinterpret_cast<const uint2*>(cs + KG_HALF + 4 * sub), sv);
+  for (int i = 0; i < KG_QP_IT; ++i) iwv[i] = iw[(size_t)r * KG_IH + (it0 + i) * 4 + wq];
 #pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int ih = it * 4 + wq;
+  for (int i = 0; i < KG_QP_IT; ++i) {
+    const int ih = (it0 + i) * 4 + wq;
     float f[8];
-    kg_unpack8(v[it], f);
+    kg_unpack8(v[i], f);
     if (roped)
 #pragma unroll
       for (int u = 0; u < 4; ++u) kg_rope(f[2 * u], f[2 * u + 1], cv[u], sv[u]);
@@ -431,7 +446,7 @@ __global__ __launch_bounds__(256) void kg_q_post_kernel(const u16* __restrict__ 
     o.y = kg_e4m3x4_signed(f[4] * inv, f[5] * inv, f[6] * inv, f[7] * inv);
     *reinterpret_cast<uint2*>(iq + ((size_t)r * KG_IH + ih) * KG_ID + 8 * m) = o;
     if (m == 0) {
-      float w = kg_bf16_to_f32(iw[(size_t)r * KG_IH + ih]);
+      float w = kg_bf16_to_f32(iwv[i]);
       w *= sc;
       w *= 0.08838834764831845f;                          // 128^-1/2
       w *= 0.17677669529663687f;                          // 32^-1/2
@@ -447,7 +462,9 @@ extern "C" int kg_q_post(const void* qb, int ldb, const void* rope, const int* p
   KG_CHECK(!full || (iq && iw && wout && kg_aligned(iq, 8)));
   KG_CHECK(kg_aligned(qb, 16) && kg_aligned(rope, 8) && kg_aligned(qmla, 16));
   if (T == 0) return 0;
-  hipLaunchKernelGGL(kg_q_post_kernel, dim3((T + 3) / 4), dim3(256), 0, (hipStream_t)stream, (const u16*)qb, ldb,
+  const long long units = (long long)T * (full ? 2 * KG_QP_UNITS : KG_QP_UNITS);
+  KG_CHECK(units < (1ll << 31) - 4);
+  hipLaunchKernelGGL(kg_q_post_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, (hipStream_t)stream, (const u16*)qb, ldb,
                      (const u16*)rope, pos, (u16*)qmla, (u8*)iq, (const u16*)iw, wout, full ? 1 : 0, T, rope_rows);
   return (int)hipGetLastError();
 }
