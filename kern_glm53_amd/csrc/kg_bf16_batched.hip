@@ -783,8 +783,11 @@ static int kg_bf16_launch(bool f32out, const void* a, const void* b, void* d, in
   KG_CHECK(a_rs % 16 == 0 && a_hs % 16 == 0 && b_rs % 16 == 0 && b_hs % 16 == 0 && d_rs % 16 == 0 &&
            d_hs % 16 == 0);
   KG_CHECK(kg_aligned(a, 16) && kg_aligned(b, 16) && kg_aligned(d, 16));
-  // 128 x 256 tiles from n = 256 on (W_UK, W_UV): a third less operand fill per output than 128 x 128
-  const int bn = n >= 256 ? 256 : 128;
+  // 128 x 256 tiles from n = 256 on (W_UK, W_UV): a third less operand fill per output than 128 x 128.  Fewer than 512
+  // of them, two per CU, leave too few loads in flight and take 128 x 128 (us, 128 x 256 / 128 x 128 with operands in
+  // HBM, 64 heads: W_UV at 16 rows 21.5 / 17.0, 300 rows (192 tiles) 28.2 / 22.0, 640 (320) 37.1 / 35.3, 1000 (512)
+  // 43.1 / 43.5; W_UK at 300 rows (384) 18.6 / 17.5, 640 (640) 26.4 / 27.8, 4096 100.5 / 106.7).
+  const int bn = n >= 256 && (long long)heads * ((m + 127) / 128) * ((n + 255) / 256) >= 512 ? 256 : 128;
   // every row offset of a tile's DMA fits the resource's 31-bit range
   KG_CHECK(a_rs >= 2ll * k && b_rs >= 2ll * k && 128ll * a_rs < (1ll << 31) && (long long)bn * b_rs < (1ll << 31));
   if (m == 0) return 0;
