@@ -16,7 +16,8 @@
 
 // ============================================================================ top-k
 
-// One 1024-thread workgroup per row.  A row of up to 65536 logits is read once, coalesced, into registers:
+// One 1024-thread workgroup per row.  A row of up to 65536 logits (V = 64 keys a thread; 16 and 32 for rows of up to
+// 16384 and 32768, whose passes then sweep no padding) is read once, coalesced, into registers:
 // element e = 4 (1024 i + t) + c of a segment (in coordinates from the 16-byte aligned origin at or below
 // the row start) is key[4 i + c] of thread t.  Longer rows are processed in segments of 65536 elements,
 // re-read on each pass.
@@ -172,7 +173,10 @@ KG_DEV void kg_tk_emit(u32* taken, u32* eqbm, bool ties, int need, int& eq_base,
 
 // MULTI = false: the row (its end within stride0 <= 65536 floats) is held in registers for every pass;
 // true: segments of 65536 are re-read on every pass (stride0 > 65536).
-template <bool MULTI>
+// V: keys a thread, the fewest that hold stride0 floats.  Short rows are bound by the passes' sweeps: with 64 keys a
+// thread, rows of 24000 add 41536 padding keys to one histogram bin.  The indexer's chain for 40 rows x 24000 (gather,
+// logits, top-k, stream rows) took 43.7 us with 64 and 33.7 with 32.
+template <bool MULTI, int V>
 __global__ __launch_bounds__(KG_TK_T) void kg_topk_kernel(const float* __restrict__ logits,
                                                            const int* __restrict__ starts,
                                                            const int* __restrict__ ends, int* __restrict__ out,
@@ -193,15 +197,16 @@ __global__ __launch_bounds__(KG_TK_T) void kg_topk_kernel(const float* __restric
   // stride0 % 4 == 0) through a resource covering the row up to its end, so a vector past it reads zeros;
   // element e of the aligned row is valid for lo <= e < hi.  (A buffer load is one instruction the
   // compiler cannot split into conditional scalar loads.)
-  const int a0 = start & ~3, lo = start - a0, hi = MULTI ? ends[r] - a0 : min(ends[r] - a0, KG_TK_SEG);
+  const int a0 = start & ~3, lo = start - a0, hi = MULTI ? ends[r] - a0 : min(ends[r] - a0, KG_TK_T * V);
   const __amdgpu_buffer_rsrc_t rrow =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(logits + (size_t)r * stride0 + a0), (short)0, hi * 4,
                                         0x00020000);
   const int nseg = MULTI ? (hi + KG_TK_SEG - 1) / KG_TK_SEG : 1;
-  u32 key[KG_TK_V];
+  u32 key[V];
+  static_assert(V % 8 == 0 && V <= KG_TK_V && (!MULTI || V == KG_TK_V), "the bitmaps hold 64 keys a thread");
   auto load = [&](int seg) {
 #pragma unroll
-    for (int i = 0; i < KG_TK_V / 4; ++i) {
+    for (int i = 0; i < V / 4; ++i) {
       const int e = seg * KG_TK_SEG + 4 * (KG_TK_T * i + t);
       const auto f = __builtin_amdgcn_raw_buffer_load_b128(rrow, (unsigned)e * 4u, 0, 0);
 #pragma unroll
@@ -215,7 +220,7 @@ __global__ __launch_bounds__(KG_TK_T) void kg_topk_kernel(const float* __restric
     for (int seg = 0; seg < nseg; ++seg) {
       if (MULTI) load(seg);
 #pragma unroll
-      for (int j = 0; j < KG_TK_V; j += 8) {
+      for (int j = 0; j < V; j += 8) {
         KgKeys8 g;
 #pragma unroll
         for (int e = 0; e < 8; ++e) g.v[e] = key[j + e];
@@ -230,6 +235,10 @@ __global__ __launch_bounds__(KG_TK_T) void kg_topk_kernel(const float* __restric
   auto mark = [&](u32 m_, u32 pm_, bool eq_taken, bool eq_marked) {
 #pragma unroll
     for (int i = 0; i < KG_TK_V / 4; ++i) {
+      if (i >= V / 4) {                           // no keys there
+        if ((t & 7) == 0) taken[(KG_TK_T * i + t) >> 3] = eqbm[(KG_TK_T * i + t) >> 3] = 0u;
+        continue;
+      }
       u32 nt = 0, ne = 0;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
@@ -307,12 +316,14 @@ extern "C" int kg_topk_prefill(const float* logits, const int* starts, const int
            stride1 == 1);
   KG_CHECK(stride0 >= 0 && stride0 % 4 == 0 && kg_aligned(logits, 16));
   if (num_rows == 0) return 0;
-  if (stride0 <= KG_TK_SEG)
-    hipLaunchKernelGGL(kg_topk_kernel<false>, dim3(num_rows), dim3(KG_TK_T), 0, (hipStream_t)stream, logits, starts,
-                       ends, out, stride0, topk, offset);
-  else
-    hipLaunchKernelGGL(kg_topk_kernel<true>, dim3(num_rows), dim3(KG_TK_T), 0, (hipStream_t)stream, logits, starts,
-                       ends, out, stride0, topk, offset);
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(num_rows), dim3(KG_TK_T), 0, (hipStream_t)stream, logits, starts, ends, out, stride0,
+                       topk, offset);
+  };
+  if (stride0 <= KG_TK_T * 16) go(kg_topk_kernel<false, 16>);
+  else if (stride0 <= KG_TK_T * 32) go(kg_topk_kernel<false, 32>);
+  else if (stride0 <= KG_TK_SEG) go(kg_topk_kernel<false, 64>);
+  else go(kg_topk_kernel<true, 64>);
   return (int)hipGetLastError();
 }
 

@@ -23,7 +23,8 @@ def run_topk(logits, starts, ends, k, num_rows=None, offset=0):
     return got, out_ref
 
 
-@pytest.mark.parametrize("case", ["mixed", "full", "ties", "unaligned", "long", "window", "k256", "specials"])
+@pytest.mark.parametrize("case", ["mixed", "full", "ties", "unaligned", "long", "window", "k256", "specials", "keys16",
+                                  "keys32", "keys64"])
 def test_topk_prefill_bit_exact(case):
     print(f"topk_prefill case={case}", flush=True)
     rng = np.random.default_rng(sum(map(ord, case)))
@@ -39,6 +40,9 @@ def test_topk_prefill_bit_exact(case):
         lens, stride0 = [40000, 40001, 40002, 5000], 40008
     elif case == "long":
         lens, stride0 = [70000, 131072, 66000, 100], 131072
+    elif case.startswith("keys"):   # the longest strides of 16 and 32 keys a thread, and one vector past them
+        lens, stride0 = {"keys16": ([16384, 16383, 2049, 9000], 16384), "keys32": ([32768, 16388, 20001], 32768),
+                         "keys64": ([32772, 32769, 30000], 32772)}[case]
     elif case == "window":
         lens, stride0 = [5000] * 8, 5120
     elif case == "specials":
