@@ -34,6 +34,7 @@ SOURCES = {
     "kg_fp8_gemm.hip": [],
     "kg_fp8_ring.hip": [],
     "kg_fp8_wfrag.hip": [],
+    "kg_fp8_wfew.hip": [],
     "kg_bf16_batched.hip": [],
     "kg_mqa_logits.hip": ["-fno-honor-nans"],
 }

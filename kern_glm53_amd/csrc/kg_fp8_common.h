@@ -18,7 +18,12 @@ struct KgFp8Args {
   u8* qsf;           // words [n / 1024][sf_rows]  (mode 2)
   int m, n, k, rows, lda, ldc, sfa_rows, groups, sf_rows;
   int m_tiles, n_tiles;
+  int few;           // experts of at most this many rows are another launch's (the fragment-order grouped modes)
 };
+
+// The few-row kernel (kg_fp8_wfew.hip) for a grouped fragment-order GEMM's experts of at most KG_WF_FEW rows.
+constexpr int KG_WF_FEW = 128;
+__attribute__((visibility("hidden"))) int kg_fp8_wfew_launch(const KgFp8Args& p, int mode, hipStream_t st);
 
 // The deep-ring dense GEMM (kg_fp8_ring.hip) over tiles of bm x bn: one of 32 x 32, 64 x 64, 64 x 128, 128 x 128,
 // 128 x 192.  Sets p.m_tiles and p.n_tiles.
@@ -118,7 +123,7 @@ KG_DEV int kg_psum_tiles(const KgFp8Args& p, int* ps, int* tp, int* wtot, int ti
       const int start = e ? ((p.psum[e - 1] + 127) >> 7) << 7 : 0;
       ps[e] = end;
       if constexpr (TAILPAIR) {
-        const int rows = end > start ? end - start : 0, rem = rows & 255;
+        const int all = end > start ? end - start : 0, rows = all > p.few ? all : 0, rem = rows & 255;
         t = ((rows >> 8) + (rem > 128)) * p.n_tiles + (rem > 0 && rem <= 128 ? p.n_tiles >> 1 : 0);
       } else {
         t = end > start ? (end - start + 255) / 256 : 0;

@@ -577,8 +577,22 @@ static int kg_wf_cus() {
   return cache[dev];
 }
 
+// The grouped GEMMs run the few-row kernel for experts of at most KG_WF_FEW rows, beside this file's for the others,
+// while `rows` leaves the experts few row slots each (with every expert padded to 128 rows: 192 slots are 64 rows on
+// average, 2048 tokens of top 8 over 256 experts; 144 slots 16 rows, 512 tokens).  gate_up 4096 x 6144, us, this kernel
+// alone / both: 24 tokens 551 / 481, 64: 952 / 779, 256: 1143 / 981, 1500: 1226 / 1107, 2048: 1223 / 1181, 3000: 1274 /
+// 1265.  down 6144 x 2048, a third of the stages per tile: 24: 281 / 258, 64: 460 / 429, 256: 586 / 560, 512: 597 / 588,
+// 768: 606 / 609, 1500: 626 / 661.
+constexpr int KG_WF_SLOTS[3] = {0, 144, 192};
 template <int MODE>
 static int kg_wf_launch(KgFp8Args& p, long long tiles, hipStream_t st) {
+  if constexpr (MODE != 0) {
+    if (p.rows <= KG_WF_SLOTS[MODE] * p.groups) {
+      p.few = KG_WF_FEW;
+      const int rc = kg_fp8_wfew_launch(p, MODE, st);
+      if (rc != 0) return rc;
+    }
+  }
   const int grid = (int)(tiles < kg_wf_cus() ? tiles : kg_wf_cus());
   if (grid <= 0) return 0;
   hipLaunchKernelGGL((kg_fp8_gemm_wfrag<MODE>), dim3(grid), dim3(256), 0, st, p);

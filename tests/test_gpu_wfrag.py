@@ -123,6 +123,28 @@ def test_fp8_gemm_psum_silu_quant_wf(case):
     assert np.array_equal(outs[0][1], outs[1][1])
 
 
+@pytest.mark.parametrize("k", [128, 640, 1536])
+@pytest.mark.parametrize("n", [512, 1536])
+def test_grouped_wf_few_rows(n, k):
+    """Experts on both sides of the few-row kernel's edges (32-row MFMA tiles, its 64- and 128-row forms) in a call whose
+    rows send those of at most 128 rows to it and the others to the persistent kernel: every byte as row-major."""
+    counts = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 200, 257] + [0, 3] * 8
+    groups, I = len(counts), n // 2
+    print(f"few rows wf n {n}, k {k}", flush=True)
+    psum, rows, a, w, sfa, sfb = grouped(counts, n, k, seed=n + k, groups=groups)
+    assert rows <= 144 * groups
+    dp, wf, outs = d(psum), frag(w), []
+    for gemm, silu, wt in ((ops.fp8_gemm_psum, ops.fp8_gemm_psum_silu_quant, w),
+                           (ops.fp8_gemm_psum_wf, ops.fp8_gemm_psum_silu_quant_wf, wf)):
+        c = filled((rows, n), SENTINEL, torch.int16)
+        gemm(a, wt, sfa, sfb, c, dp, n=n, k=k, rows=rows, lda=k, ldc=n, sfa_rows=rows, groups=groups)
+        q, sf = filled((rows, I), 0x5c), filled((ref.sf_words(I) * rows * 4,), 0x5d)
+        silu(a, wt, sfa, sfb, dp, q, sf, n=n, k=k, rows=rows, lda=k, sfa_rows=rows, sf_rows=rows, groups=groups)
+        outs.append((h(c, np.uint16), h(q, np.uint8), h(sf, np.uint8)))
+    for x, y in zip(*outs):
+        assert np.array_equal(x, y)
+
+
 def test_moe_wf_full_size():
     """The bench's routed MoE (16384 tokens x top-8 over 256 experts, Zipf(1.1)): the fragment-order gate_up
     (fused SiLU-mul-quant) and down GEMMs equal the row-major ones on every byte."""
