@@ -18,12 +18,37 @@ struct KgFp8Args {
   u8* qsf;           // words [n / 1024][sf_rows]  (mode 2)
   int m, n, k, rows, lda, ldc, sfa_rows, groups, sf_rows;
   int m_tiles, n_tiles;
-  int few;           // experts of at most this many rows are another launch's (the fragment-order grouped modes)
+  int few;           // the experts of at most this many rows may be another launch's (fragment-order grouped modes)
 };
 
-// The few-row kernel (kg_fp8_wfew.hip) for a grouped fragment-order GEMM's experts of at most KG_WF_FEW rows.
-constexpr int KG_WF_FEW = 128;
+// The few-row kernel (kg_fp8_wfew.hip) for a grouped fragment-order GEMM: its experts of at most p.few (<= 128) rows,
+// or with p.few = 0 every expert's rows, 128 at a time.
 __attribute__((visibility("hidden"))) int kg_fp8_wfew_launch(const KgFp8Args& p, int mode, hipStream_t st);
+
+// Whether the experts of at most p.few rows go to the few-row kernel (wave-uniform; both kernels ask, `lane` is 0 .. 63):
+// when no expert has more, or half of those with rows have at most p.few / 2.  Experts that straddle p.few cost a round
+// of each kernel (256 experts of 120 rows on average, 4096 x 6144: 1256 us in one kernel, 1340 in both), which pays
+// where most of the weights stream through the few-row kernel at its best.
+KG_DEV bool kg_wf_split(const KgFp8Args& p, int lane) {
+  int live = 0, small = 0, large = 0;
+  for (int e0 = 0; e0 < p.groups; e0 += 256) {
+    int end[4], prev[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int e = e0 + x * 64 + lane;
+      end[x] = e < p.groups ? p.psum[e] : 0;
+      prev[x] = e > 0 && e < p.groups ? p.psum[e - 1] : 0;
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int rows = end[x] - (((prev[x] + 127) >> 7) << 7);   // past the last expert: at most 0
+      live += __popcll(__ballot(rows > 0));
+      small += __popcll(__ballot(rows > 0 && rows <= p.few >> 1));
+      large += __popcll(__ballot(rows > p.few));
+    }
+  }
+  return large == 0 || 2 * small >= live;
+}
 
 // The deep-ring dense GEMM (kg_fp8_ring.hip) over tiles of bm x bn: one of 32 x 32, 64 x 64, 64 x 128, 128 x 128,
 // 128 x 192.  Sets p.m_tiles and p.n_tiles.
@@ -113,7 +138,9 @@ KG_DEV KgPTile kg_ptile(const KgFp8Args& p, const int* tp, const int* ps, int to
 // n_tiles / 2 tiles (each a pair of column tiles); tp[] is then the exclusive prefix of the tile counts.
 template <bool TAILPAIR = false>
 KG_DEV int kg_psum_tiles(const KgFp8Args& p, int* ps, int* tp, int* wtot, int tid, int lane, int wave) {
-  int part = 0, tl[4];
+  int part = 0, tl[4], few = 0;                 // few: experts of at most this many rows are the few-row kernel's
+  if constexpr (TAILPAIR)
+    if (p.few && kg_wf_split(p, lane)) few = p.few;
 #pragma unroll
   for (int x = 0; x < 4; ++x) {
     const int e = tid * 4 + x;
@@ -123,7 +150,7 @@ KG_DEV int kg_psum_tiles(const KgFp8Args& p, int* ps, int* tp, int* wtot, int ti
       const int start = e ? ((p.psum[e - 1] + 127) >> 7) << 7 : 0;
       ps[e] = end;
       if constexpr (TAILPAIR) {
-        const int all = end > start ? end - start : 0, rows = all > p.few ? all : 0, rem = rows & 255;
+        const int all = end > start ? end - start : 0, rows = all > few ? all : 0, rem = rows & 255;
         t = ((rows >> 8) + (rem > 128)) * p.n_tiles + (rem > 0 && rem <= 128 ? p.n_tiles >> 1 : 0);
       } else {
         t = end > start ? (end - start + 255) / 256 : 0;

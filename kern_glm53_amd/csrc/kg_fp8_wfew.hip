@@ -1,4 +1,5 @@
-// Grouped fp8 GEMMs with the weights in fragment order, for the experts of at most 128 rows: the same two grouped
+// Grouped fp8 GEMMs with the weights in fragment order, for the experts of at most 128 rows (and in small calls for
+// every expert, 128 rows at a time; the rule is in kg_fp8_wfrag.hip): the same two grouped
 // modes and the same arithmetic as kg_fp8_gemm_wfrag (m-grouped psum; m-grouped gate_up with the fused SiLU-mul-quant
 // epilogue), bit for bit.
 //
@@ -37,11 +38,26 @@ __global__ __launch_bounds__(256, 2) void kg_fp8_gemm_wfew(const KgFp8Args p) {
   __shared__ float xam[4][128];
   __shared__ u8 xe[128];
 
-  const int g = (int)blockIdx.x / p.n_tiles, nt = (int)blockIdx.x - g * p.n_tiles;
-  const int start = g ? ((p.psum[g - 1] + 127) >> 7) << 7 : 0, m_end = min(p.psum[g], p.rows), nrows = m_end - start;
-  if (nrows <= 0 || p.psum[g] - start > KG_WF_FEW) return;     // uniform: the persistent kernel's
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int unit = (int)blockIdx.x / p.n_tiles, nt = (int)blockIdx.x - unit * p.n_tiles;
+  int g = unit, start, m_end;
+  if (p.few == 0) {                                            // unit: the 128 rows from `start`, of the expert there
+    start = unit << 7, g = -1;
+    for (int e0 = 0; e0 < p.groups && g < 0; e0 += 64) {
+      const int e = e0 + lane;
+      bool here = false;
+      if (e < p.groups) here = (e ? ((p.psum[e - 1] + 127) >> 7) << 7 : 0) <= start && start < p.psum[e];
+      const unsigned long long m = __ballot(here);
+      if (m) g = e0 + __builtin_ctzll(m);
+    }
+    if (g < 0) return;                                         // uniform: no expert's rows
+    m_end = min(p.psum[g], start + 128);
+  } else {                                                     // unit: an expert of at most p.few rows
+    start = g ? ((p.psum[g - 1] + 127) >> 7) << 7 : 0, m_end = min(p.psum[g], p.rows);
+    if (m_end <= start || p.psum[g] - start > p.few || !kg_wf_split(p, lane)) return;   // uniform: the persistent kernel's
+  }
+  const int nrows = m_end - start;
   const int half = p.n >> 1, kw = (p.k + 511) >> 9, KB = p.k >> 7, KS = kw << 2, n0 = nt * CN;
 
   const __amdgpu_buffer_rsrc_t ra = kg_rsrc(p.a + (size_t)start * p.lda, (long long)(nrows - 1) * p.lda + p.k);
@@ -270,7 +286,7 @@ template __global__ void kg_fp8_gemm_wfew<1>(const KgFp8Args);
 template __global__ void kg_fp8_gemm_wfew<2>(const KgFp8Args);
 
 int kg_fp8_wfew_launch(const KgFp8Args& p, int mode, hipStream_t st) {
-  const dim3 grid((unsigned)(p.groups * p.n_tiles));
+  const dim3 grid((unsigned)((p.few ? p.groups : p.rows >> 7) * p.n_tiles));
   if (mode == 1) hipLaunchKernelGGL((kg_fp8_gemm_wfew<1>), grid, dim3(256), 0, st, p);
   else hipLaunchKernelGGL((kg_fp8_gemm_wfew<2>), grid, dim3(256), 0, st, p);
   return (int)hipGetLastError();

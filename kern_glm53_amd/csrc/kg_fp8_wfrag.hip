@@ -577,18 +577,29 @@ static int kg_wf_cus() {
   return cache[dev];
 }
 
-// The grouped GEMMs run the few-row kernel for experts of at most KG_WF_FEW rows, beside this file's for the others,
-// while `rows` leaves the experts few row slots each (with every expert padded to 128 rows: 192 slots are 64 rows on
-// average, 2048 tokens of top 8 over 256 experts; 144 slots 16 rows, 512 tokens).  gate_up 4096 x 6144, us, this kernel
-// alone / both: 24 tokens 551 / 481, 64: 952 / 779, 256: 1143 / 981, 1500: 1226 / 1107, 2048: 1223 / 1181, 3000: 1274 /
-// 1265.  down 6144 x 2048, a third of the stages per tile: 24: 281 / 258, 64: 460 / 429, 256: 586 / 560, 512: 597 / 588,
-// 768: 606 / 609, 1500: 626 / 661.
+// Which kernel takes a grouped GEMM's experts (us, this file's kernel alone / with the rule; E experts of n x k).
+//   * Calls of at most one workgroup a CU over their 128-row blocks: the few-row kernel takes every block, in one launch
+//     whose chain of K blocks is shorter (E 8, 4096 x 6144, 20 rows each 65 / 43; four experts, three of 8 rows and one
+//     of 200, 61 / 45; E 8, 1024 x 1024 20 / 12).
+//   * Weights of KG_WF_SPLIT_BYTES or more, and `rows` that leave the experts few row slots each (with every expert
+//     padded to 128 rows: 192 slots are 64 rows on average, 2048 tokens of top 8 over 256 experts; 144 slots 16 rows,
+//     512 tokens): two launches, the few-row kernel for the experts of at most KG_WF_FEW rows, this file's for the
+//     others, if kg_wf_split finds most experts small enough.  gate_up 4096 x 6144, E 256: 24 tokens 669 / 568, 64:
+//     1057 / 857, 512: 1143 / 991, 1500: 1157 / 1044, 2048: 1167 / 1078 (3000: 1274 / 1265).  down 6144 x 2048, a third
+//     of the stages per tile: 24: 330 / 303, 64: 503 / 468, 256: 581 / 551, 512: 592 / 571; its experts of 60 rows are
+//     no faster in the few-row kernel (606 / 664), so it takes those of at most 32.
+//   * Below those bytes the two launches, one after the other, cost more than they save once an expert is on either
+//     side (gate_up, E 8, 4096 x 6144 66 / 111, E 32, 1024 x 1024 22 / 33; down, E 32, 4096 x 6144 of 20 rows on average
+//     146 / 195), and this file's kernel runs alone.  A few-row launch that finds nothing to do costs 8 us at E 256.
 constexpr int KG_WF_SLOTS[3] = {0, 144, 192};
+constexpr int KG_WF_FEW[3] = {0, 32, 128};
+constexpr long long KG_WF_SPLIT_BYTES[3] = {0, 1536ll << 20, 768ll << 20};
 template <int MODE>
 static int kg_wf_launch(KgFp8Args& p, long long tiles, hipStream_t st) {
   if constexpr (MODE != 0) {
-    if (p.rows <= KG_WF_SLOTS[MODE] * p.groups) {
-      p.few = KG_WF_FEW;
+    if ((long long)(p.rows >> 7) * p.n_tiles <= kg_wf_cus()) return kg_fp8_wfew_launch(p, MODE, st);
+    if (p.rows <= KG_WF_SLOTS[MODE] * p.groups && (long long)p.groups * p.n * p.k >= KG_WF_SPLIT_BYTES[MODE]) {
+      p.few = KG_WF_FEW[MODE];
       const int rc = kg_fp8_wfew_launch(p, MODE, st);
       if (rc != 0) return rc;
     }

@@ -29,3 +29,20 @@ def filled(shape, value, dtype=torch.uint8) -> torch.Tensor:
 def bf16_bits(x: torch.Tensor) -> np.ndarray:
     """bf16 tensor (any device) -> uint16 numpy bits."""
     return x.detach().cpu().contiguous().view(torch.int16).numpy().view(np.uint16)
+
+
+def fastest(calls, passes: int = 20, rounds: int = 7) -> list[float]:
+    """Microseconds a pass of each call: the least of `rounds` timings of `passes` passes, the calls in turn."""
+    best = [float("inf")] * len(calls)
+    for call in calls:
+        call()
+    for _ in range(rounds):
+        for i, call in enumerate(calls):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(passes):
+                call()
+            b.record()
+            b.synchronize()
+            best[i] = min(best[i], a.elapsed_time(b) * 1e3 / passes)
+    return best

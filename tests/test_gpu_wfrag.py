@@ -14,7 +14,7 @@ import torch
 
 from kern_glm53_amd import ops, synth
 from oracle import ref
-from tests._gpu import DEV, d, filled, h
+from tests._gpu import DEV, d, fastest, filled, h
 from tests.test_gpu_gemm import SENTINEL, check, model_on_rows, quant_act, quant_weight, sample_rows
 
 pytestmark = pytest.mark.gpu
@@ -123,16 +123,19 @@ def test_fp8_gemm_psum_silu_quant_wf(case):
     assert np.array_equal(outs[0][1], outs[1][1])
 
 
+FEW = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 200, 257]
+
+
 @pytest.mark.parametrize("k", [128, 640, 1536])
 @pytest.mark.parametrize("n", [512, 1536])
 def test_grouped_wf_few_rows(n, k):
-    """Experts on both sides of the few-row kernel's edges (32-row MFMA tiles, its 64- and 128-row forms) in a call whose
-    rows send those of at most 128 rows to it and the others to the persistent kernel: every byte as row-major."""
-    counts = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 200, 257] + [0, 3] * 8
+    """Experts on both sides of the few-row kernel's edges (32-row MFMA tiles, its 64- and 128-row forms) in a call small
+    enough for it to take every expert in 128-row blocks: every byte as row-major."""
+    counts = FEW + [0, 3] * 8
     groups, I = len(counts), n // 2
     print(f"few rows wf n {n}, k {k}", flush=True)
     psum, rows, a, w, sfa, sfb = grouped(counts, n, k, seed=n + k, groups=groups)
-    assert rows <= 144 * groups
+    assert rows // 128 * (n // 256) <= 256
     dp, wf, outs = d(psum), frag(w), []
     for gemm, silu, wt in ((ops.fp8_gemm_psum, ops.fp8_gemm_psum_silu_quant, w),
                            (ops.fp8_gemm_psum_wf, ops.fp8_gemm_psum_silu_quant_wf, wf)):
@@ -143,6 +146,67 @@ def test_grouped_wf_few_rows(n, k):
         outs.append((h(c, np.uint16), h(q, np.uint8), h(sf, np.uint8)))
     for x, y in zip(*outs):
         assert np.array_equal(x, y)
+
+
+def big_grouped(counts, n, k, seed):
+    """grouped() made on the device: experts of `counts` rows in a capacity of just their 128-row blocks."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    codes = lambda *s: torch.randint(0, 0x7f, s, generator=g, device=DEV, dtype=torch.uint8)
+    sf = lambda groups, r: torch.randint(118, 127, (groups * ref.sf_words(k) * r * 4,), generator=g, device=DEV,
+                                         dtype=torch.uint8)
+    psum = ref.moe_psum(np.asarray(counts, np.int32), len(counts))
+    rows = int((psum[-1] + 127) // 128 * 128)
+    return d(psum), rows, codes(rows, k), codes(len(counts) * n, k), sf(1, rows), sf(len(counts), n)
+
+
+def split(counts, few):
+    """Whether the two fragment-order kernels share the experts (those of at most `few` rows to the few-row one)."""
+    live = [c for c in counts if c]
+    return max(live) <= few or 2 * sum(c <= few // 2 for c in live) >= len(live)
+
+
+@pytest.mark.parametrize("shared", [True, False])
+def test_grouped_wf_split_experts(shared):
+    """Weights large enough (1.8 GB) for the two kernels to share the experts, on both sides of the edges between them
+    (32 rows, 128 with the fused epilogue) and of the few-row kernel's MFMA tiles, with most experts small enough for
+    that or not: every byte as row-major."""
+    counts = ([1, 15, 16, 17, 31, 32, 33, 64, 65, 127, 128, 129, 200, 257] + [0, 3, 9, 16] * 7) * 24 if shared else \
+        (FEW + [0, 3, 0, 7]) * 51
+    counts, n, k = counts + [5] * (1024 - len(counts)), 1536, 1152
+    groups, I = len(counts), n // 2
+    print(f"split wf {groups} experts, shared {shared}", flush=True)
+    psum, rows, a, w, sfa, sfb = big_grouped(counts, n, k, seed=5)
+    assert rows <= 144 * groups and groups * n * k >= 1536 << 20
+    assert split(counts, 32) == split(counts, 128) == shared
+    wf, outs = frag(w), []
+    for gemm, silu, wt in ((ops.fp8_gemm_psum, ops.fp8_gemm_psum_silu_quant, w),
+                           (ops.fp8_gemm_psum_wf, ops.fp8_gemm_psum_silu_quant_wf, wf)):
+        c = filled((rows, n), SENTINEL, torch.int16)
+        gemm(a, wt, sfa, sfb, c, psum, n=n, k=k, rows=rows, lda=k, ldc=n, sfa_rows=rows, groups=groups)
+        q, sf = filled((rows, I), 0x5c), filled((ref.sf_words(I) * rows * 4,), 0x5d)
+        silu(a, wt, sfa, sfb, psum, q, sf, n=n, k=k, rows=rows, lda=k, sfa_rows=rows, sf_rows=rows, groups=groups)
+        outs.append((c, q, sf))
+    for x, y in zip(*outs):
+        assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("counts,n,k", [([8, 8, 8, 200], 4096, 6144),                   # one workgroup a CU
+                                        ([60] * 30 + [130, 150], 1024, 1024),
+                                        ([128] * 7 + [129], 4096, 6144),
+                                        ([60] * 12 + [200] * 4, 6144, 2048)])           # neither form: one kernel alone
+def test_grouped_wf_mixed_experts_time(counts, n, k):
+    """A call with experts on both sides of 128 rows whose weights are too few to stream for long is one launch: two, one
+    after the other, took 1.4 to 1.7 times the row-major kernel's time (one launch 0.7 to 1.05 times)."""
+    groups = len(counts)
+    psum, rows, a, w, sfa, sfb = big_grouped(counts, n, k, seed=groups)
+    q, sf = filled((rows, n // 2), 0), filled((ref.sf_words(n // 2) * rows * 4,), 0)
+    wf = frag(w)
+    calls = [lambda fn=fn, wt=wt: fn(a, wt, sfa, sfb, psum, q, sf, n=n, k=k, rows=rows, lda=k, sfa_rows=rows, sf_rows=rows,
+                                     groups=groups)
+             for fn, wt in ((ops.fp8_gemm_psum_silu_quant, w), (ops.fp8_gemm_psum_silu_quant_wf, wf))]
+    t_row, t_wf = fastest(calls)
+    print(f"mixed wf {groups} experts {n} x {k}: row-major {t_row:.1f} us, fragment order {t_wf:.1f}", flush=True)
+    assert t_wf <= 1.25 * t_row
 
 
 def test_moe_wf_full_size():
