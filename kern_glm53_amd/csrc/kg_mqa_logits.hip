@@ -6,10 +6,10 @@
 // rounds only differently in the f32 head summation order.
 //
 // Design: a workgroup of 8 wave64s owns 8 query rows (one per wave, its 32 heads as the rows of the MFMA
-// tiles, kept in registers for the whole key loop) and walks a slice of the union of their key ranges (all of it
-// when there are rows enough to fill the chip) 64 keys at a time.  A key block (64 keys x 128 bytes, and the 64 key scales) is copied HBM -> LDS by
-// buffer_load ... lds into one of three LDS stages (XOR-swizzled rows as in the GEMMs) and consumed as
-// 2 key tiles x 2 K halves of v_mfma_scale_f32_32x32x64_f8f6f4 (unit scales).  Each lane of a 32x32
+// tiles, kept in registers for the whole key loop) and walks a slice of the union of their key ranges (all of
+// it when there are rows enough to fill the chip) 64 keys at a time.  A key block (64 keys x 128 bytes, and the 64 key
+// scales) is copied HBM -> LDS by buffer_load ... lds into one of three LDS stages (XOR-swizzled rows as in the GEMMs)
+// and consumed as 2 key tiles x 2 K halves of v_mfma_scale_f32_32x32x64_f8f6f4 (unit scales).  Each lane of a 32x32
 // score tile holds one key and 16 of the 32 heads: relu and the head weight (fma) give a partial head
 // sum, v_permlane32_swap pairs the two tiles' halves, one add finishes both tiles' sums, then the key
 // scale and one store of 64 consecutive logits.  30 KB of LDS and 127 VGPRs: 2 workgroups per CU.  Eight
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(512, 2) void kg_mqa_logits_kernel(const u8* __restr
                                                                const unsigned* __restrict__ ks,
                                                                const unsigned* __restrict__ ke,
                                                                float* __restrict__ logits, int num_q, int num_kv,
-                                                               int stride, int slice) {
+                                                               int stride, int slice, int slices) {
   // a stage: 64 keys x 128 bytes, then 8 regions of 64 key scales (one per wave; region 0 is read)
   constexpr int BK = 64, TB = BK / 32, KEYB = BK * 128, STAGE = KEYB + 2048;
   __shared__ __attribute__((aligned(1024))) u8 st0[STAGE];
@@ -63,11 +63,17 @@ __global__ __launch_bounds__(512, 2) void kg_mqa_logits_kernel(const u8* __restr
   unsigned kmin = srange[0][0], kmax = srange[1][0];
 #pragma unroll
   for (int i = 1; i < NW; ++i) kmin = min(kmin, srange[0][i]), kmax = max(kmax, srange[1][i]);
-  // this workgroup's slice of the union: keys [kmin + y slice, + slice)
+  // this workgroup's slice of the union: keys [kmin + y slice, + slice), in longer slices (of 6 j + 1 blocks too) where
+  // the rows straddle packed sequences and `slices` (gridDim.y) of them do not reach its end
   kmin = __builtin_amdgcn_readfirstlane(kmin);
   kmax = __builtin_amdgcn_readfirstlane(kmax);
+  if (kmin >= kmax) return;                          // uniform: no live key in the workgroup
+  if (kmax - kmin > (unsigned)slices * (unsigned)slice) {
+    const unsigned need = ((kmax - kmin + 63) / 64 + (unsigned)slices - 1) / (unsigned)slices;
+    slice = (int)((need + 4) / 6 * 6 + 1) * 64;
+  }
   const unsigned skip = blockIdx.y * (unsigned)slice;
-  if (kmin >= kmax || kmax - kmin <= skip) return;   // uniform: no live key in the slice
+  if (kmax - kmin <= skip) return;                   // uniform: no live key in the slice
   kmin += skip;
   kmax = min(kmax, kmin + (unsigned)slice);
   bool any_row = false;                              // rows of several packed sequences leave gaps
@@ -216,25 +222,28 @@ __global__ __launch_bounds__(512, 2) void kg_mqa_logits_kernel(const u8* __restr
   __builtin_amdgcn_s_waitcnt(0);                 // no DMA into LDS may be in flight at exit
 }
 
-// Key blocks (of 64) per workgroup, 6 j + 1 (the main loop's step, so that no block of a full slice is wasted).
+// Key blocks (of 64) per slice, 6 j + 1 (the main loop's step, so that no block of a full slice is wasted).
 // The chip holds 512 workgroups, two per CU.  A key block takes a workgroup alone on its CU 0.45-0.55 us, one of two
-// 0.95 us, and a workgroup costs about 4.5 us besides (its queries, its first keys' latency, its last stores).  Of
-// the slices that just fill half the slots (one workgroup a CU) or 1 .. 8 times all of them, the one with the least
-// time by that.  Measured (us, rows x context, one workgroup per 8 rows before / sliced): 40 x 24000 of two
-// sequences 357 / 11.4, 1024 x 65536 516 / 254, 1024 x 8192 68 / 44, 200 x 30000 220 / 32, 1 x 65536 481 / 7.5.
-// From 2048 groups on (16384 rows) the slots are full without slices, and a group keeps its whole range.
-// `blocks` is the longest row's; groups whose rows span packed sequences walk more.
+// 0.95 us, and a workgroup costs about 4.5 us besides (its queries, its first keys' latency, its last stores).  Those of
+// later rounds pass beside the other workgroup's work and buy a better balance over rows of unequal length, but the
+// shortest slices' from about the fifth round on, 1.2 us a round (4000 rows of two sequences of 2000 keys: one round of
+// whole ranges 31.9 us, five of 7 blocks 29.6; 13820 rows of 20 sequences of 691 keys: four rounds of whole ranges 45.3,
+// seven of 7 blocks 48.7; 1024 x 65536: one round of 259 blocks 7 us more than six of 43).  Of the slices that just
+// fill half the slots (one workgroup a CU) or 1 .. 8 times all of them, the one with the least time by that.  Measured
+// (us, rows x context, one workgroup per 8 rows before / sliced): 40 x 24000 of two sequences 357 / 11.4, 1024 x 65536
+// 516 / 254, 1024 x 8192 68 / 44, 200 x 30000 220 / 32, 1 x 65536 481 / 7.5.  `blocks` is the longest row's; groups
+// whose rows span packed sequences walk more.
 static int kg_mqa_slice(long long groups, long long blocks) {
-  long long best = blocks;
+  long long best = blocks < 7 ? 7 : blocks;
   double least = 1e30;
   for (int w = 0; w <= 8; ++w) {
     const long long parts = (w ? 512ll * w : 256) / groups;
     if (parts < 1) continue;
-    const long long need = (blocks + parts - 1) / parts, slice = need <= 1 ? 1 : (need + 4) / 6 * 6 + 1;
-    const double t = w ? 0.95 * w * slice + 4.5 : 0.55 * slice + 4.5;
+    const long long need = (blocks + parts - 1) / parts, slice = need <= 7 ? 7 : (need + 4) / 6 * 6 + 1;
+    const double t = w ? 0.95 * w * slice + (w > 4 && slice == 7 ? 1.2 * (w - 4) : 0.0) + 4.5 : 0.55 * slice + 4.5;
     if (t < least) least = t, best = slice;
   }
-  return (int)(best < 7 ? 7 : best);
+  return (int)best;
 }
 
 extern "C" int kg_mqa_logits(const void* q, const void* kv, const float* ksf, const float* w, const unsigned* ks,
@@ -245,9 +254,15 @@ extern "C" int kg_mqa_logits(const void* q, const void* kv, const float* ksf, co
   KG_CHECK((long long)num_kv * 128 < (1ll << 31) && (long long)stride * 4 < (1ll << 31));
   if (num_q == 0) return 0;
   const int groups = (num_q + 7) / 8, blocks = num_kv > 0 ? (num_kv + 63) / 64 : 1;
-  const int slice = kg_mqa_slice(groups, (min(num_kv, stride) + 63) / 64);
-  hipLaunchKernelGGL(kg_mqa_logits_kernel, dim3(groups, (blocks + slice - 1) / slice), dim3(512), 0,
-                     (hipStream_t)stream, (const u8*)q, (const u8*)kv, ksf, w, ks, ke, logits, num_q, num_kv, stride,
-                     slice * 64);
+  const int row_blocks = (min(num_kv, stride) + 63) / 64, slice = kg_mqa_slice(groups, row_blocks);
+  // Workgroups for a row's slices, or as many as fill the slots and a quarter, up to all slices of the stream; groups
+  // that straddle packed sequences make their slices longer where these do not reach.  (A workgroup for every slice of
+  // the stream, most of them without keys: 13814 rows of 20 sequences of 691 keys 92 us, 16384 of 16 of 1024 82; so 44
+  // and 63.  Without the quarter 40 rows of two sequences of 24000 keys take 2 us more, in the group that straddles
+  // them; with the slots filled twice, 2000 rows of 8 of 700 15.7, so 12.4.)
+  const int parts = max(max((row_blocks + slice - 1) / slice, 640 / groups), 1);
+  const int slices = min((blocks + slice - 1) / slice, parts);
+  hipLaunchKernelGGL(kg_mqa_logits_kernel, dim3(groups, slices), dim3(512), 0, (hipStream_t)stream, (const u8*)q,
+                     (const u8*)kv, ksf, w, ks, ke, logits, num_q, num_kv, stride, slice * 64, slices);
   return (int)hipGetLastError();
 }

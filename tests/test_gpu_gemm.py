@@ -17,7 +17,7 @@ import torch
 
 from kern_glm53_amd import ops, synth
 from oracle import ref
-from tests._gpu import DEV, bf16_bits, d, filled, h
+from tests._gpu import DEV, bf16_bits, d, fastest, filled, h
 
 pytestmark = pytest.mark.gpu
 
@@ -622,6 +622,51 @@ def test_mqa_logits_key_slices(num_q, num_kv):
         ke[2::3] = rng.integers(0, 200, len(ke[2::3]))                # its start only (a gap between the two)
     out = run_mqa(q8, k8, ksf, w, ks, ke, (num_kv + 63) // 64 * 64)
     check_mqa(out, q8, k8, ksf, w, ks, ke, (num_kv + 63) // 64 * 64)
+
+
+@pytest.mark.parametrize("num_q,seqs,ctx", [(5128, 20, 257), (5200, 9, 1100), (1030, 7, 513)])
+def test_mqa_logits_straddling_groups(num_q, seqs, ctx):
+    """Packed sequences whose edges fall inside groups of 8 rows, with fewer workgroups a group than the group's keys have
+    slices (5128 and 5200 rows; longer slices) and with enough: each sequence's logits as in a call of its own."""
+    print(f"mqa straddling {num_q} rows of {seqs}", flush=True)
+    g = synth.generator(31, "cuda")
+    codes = lambda *s: torch.randint(0, 0x78, s, generator=g, device=DEV, dtype=torch.uint8)
+    iq, kg = codes(num_q, 32, 128), codes(seqs * ctx, 128)
+    ksf = torch.exp2(torch.randint(-8, 0, (seqs * ctx,), generator=g, device=DEV).float())
+    w = torch.randn(num_q, 32, generator=g, device=DEV)
+    stride, row = (ctx + 255) // 256 * 256, 0
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    lens = [num_q // seqs + (i < num_q % seqs) for i in range(seqs)]
+    ks = i32([i * ctx for i, n in enumerate(lens) for _ in range(n)])
+    klen = i32([max(1, k) for n in lens for k in range(ctx - n + 1, ctx + 1)])
+    out = torch.full((num_q, stride), -12345.0, device=DEV)
+    ops.mqa_logits(iq, kg, ksf, w, ks, ks + klen, out, num_q, seqs * ctx, stride)
+    for i, n in enumerate(lens):
+        own, sl, keys = torch.full((n, stride), -12345.0, device=DEV), slice(row, row + n), slice(i * ctx, (i + 1) * ctx)
+        ops.mqa_logits(iq[sl], kg[keys], ksf[keys].clone(), w[sl].clone(), torch.zeros_like(klen[sl]), klen[sl].clone(), own,
+                       n, ctx, stride)
+        assert torch.equal(out[sl], own), f"sequence {i}"
+        row += n
+
+
+@pytest.mark.parametrize("num_q,seqs,ctx", [(13814, 20, 691), (1024, 64, 1024)])
+def test_mqa_logits_packed_time(num_q, seqs, ctx):
+    """Many short sequences take about the time of the same rows with the same key counts over one sequence's keys: no
+    workgroups for the other sequences' keys (which took 2.1 and 1.8 times it)."""
+    g = synth.generator(21, "cuda")
+    codes = lambda *s: torch.randint(0, 0x78, s, generator=g, device=DEV, dtype=torch.uint8)
+    iq, kg = codes(num_q, 32, 128), codes(seqs * ctx, 128)
+    ksf, w = torch.ones(seqs * ctx, device=DEV), torch.randn(num_q, 32, generator=g, device=DEV)
+    lens = [num_q // seqs + (i < num_q % seqs) for i in range(seqs)]
+    ks = torch.tensor([i * ctx for i, n in enumerate(lens) for _ in range(n)], dtype=torch.int32, device=DEV)
+    klen = torch.tensor([k for n in lens for k in range(ctx - n + 1, ctx + 1)], dtype=torch.int32, device=DEV)
+    stride = (ctx + 255) // 256 * 256
+    logits = torch.empty(num_q, stride, dtype=torch.float32, device=DEV)
+    zero, ke = torch.zeros_like(ks), ks + klen
+    one, packed = fastest([lambda: ops.mqa_logits(iq, kg, ksf, w, zero, klen, logits, num_q, ctx, stride),
+                           lambda: ops.mqa_logits(iq, kg, ksf, w, ks, ke, logits, num_q, seqs * ctx, stride)])
+    print(f"mqa {num_q} rows: one sequence {one:.1f} us, {seqs} sequences {packed:.1f}", flush=True)
+    assert packed <= 1.4 * one
 
 
 def test_mqa_logits_causal_chunk():
