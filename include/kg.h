@@ -27,10 +27,11 @@ extern "C" {
  * f32 accumulation.  a: e4m3 [rows][lda]; w: e4m3 [n][k]; sfa: words [k/512][sfa_rows]; sfb: words
  * [k/512][n] (one word per weight row); c: bf16 [rows][ldc], columns [n, ldc) untouched.
  * Requires k % 128 == 0, m <= rows <= sfa_rows, n <= ldc, k <= lda, lda % 16 == 0, ldc % 4 == 0, a and w
- * 16-byte aligned, c 8-byte aligned; with 256 or more tiles of 256 x 256 (the persistent kernel, taken
- * when n % 8 == 0, ldc % 8 == 0 and c is 16-byte aligned) also rows * lda and rows * ldc * 2 below 2^31;
+ * 16-byte aligned, c 8-byte aligned; with 256 or more tiles of 256 x 256, where n % 8 == 0, ldc % 8 == 0, c is 16-byte
+ * aligned and rows * ldc * 2 is below 2^31 (the persistent kernel can store them), also rows * lda below 2^31;
  * always n * k, 256 * lda and the scale arrays' bytes (4 ceil(k/512) sfa_rows, 4 ceil(k/512) n) below
- * 2^31 (the byte ranges of the kernels' buffer resources and their 32-bit offsets). */
+ * 2^31 (the byte ranges of the kernels' buffer resources and their 32-bit offsets).  The kernel and tile shape are picked
+ * by size; the outputs do not depend on them. */
 int kg_fp8_gemm(const void* a, const void* w, const void* sfa, const void* sfb, void* c, int m, int n, int k,
                 int rows, int lda, int ldc, int sfa_rows, void* stream);
 

@@ -94,7 +94,7 @@ KG_DEV void kg_fp8_epilogue(const KgFp8Args& p, v16f (&acc)[BN / 64][BM / 64], i
   }
 }
 
-// Dense GEMMs of more than one and at most two 128 x 128 tiles per CU: one tile per workgroup, K blocks of 128 through
+// Dense GEMMs that fill two 128 x 128 tiles per CU best: one tile per workgroup, K blocks of 128 through
 // two LDS stages, two workgroups per CU (1700 x 4096 x 6144: 448 tiles in 57.7 us, against 62.1 as two rounds of the
 // deep-ring kernel).
 __global__ __launch_bounds__(256, 2) void kg_fp8_gemm_tile(const KgFp8Args p) {
@@ -755,29 +755,36 @@ extern "C" int kg_fp8_gemm(const void* a, const void* w, const void* sfa, const 
   p.m = m, p.n = n, p.k = k, p.rows = rows, p.lda = lda, p.ldc = ldc, p.sfa_rows = sfa_rows, p.groups = 1;
   hipStream_t st = (hipStream_t)stream;
   // The kernel and tile shape with the least estimated time: rounds of one tile per slot, each a fixed part and a part
-  // per K block of 128.  The parts are fitted to timings (weights from HBM) of M = 1 .. 4100 at seven N x K from 2752 x
-  // 6144 to 24576 x 6144; over those 130 sizes the pick is within 4% of the best kernel but for one at 12%, and the
-  // deep-ring kernels run 1.56 times as fast as the two others alone (geometric mean).
+  // per K block of 128, and the persistent kernel's start.  The parts are fitted to timings (weights from HBM) of M = 1
+  // .. 16384 at fourteen N x K from 512 x 512 to 24576 x 6144.  Over those 520 sizes the pick is 0.5% behind the best
+  // kernel on average, 25% at most (16384 x 512 x 512, 12.4 us against 9.9), and nowhere more than 1.5% slower than the
+  // last two kernels alone (256 x 256 from 256 such tiles on), over which it gains 1.32 times (geometric mean).  The 256
+  // x 256 tiles are the best of fewer than 256, too, where they take one round and the others three (5000 x 2752 x 6144
+  // 72 us, 102 in 128 x 192), and about even with two rounds of 128 x 192 (420 x 24576 x 6144 79 and 78.5 us, 67 and 70
+  // with the weights in the last-level cache).
   struct Shape {
     int bm, bn, per_cu;
-    float fixed, block;                          // us
+    float fixed, block, start;                   // us
   };
-  static const Shape shapes[] = {
-      {32, 32, 1, 2.2f, 0.165f},   {64, 64, 1, 2.1f, 0.30f},   {64, 128, 1, 2.2f, 0.40f}, {128, 128, 1, 3.3f, 0.54f},
-      {128, 192, 1, 4.4f, 0.68f},  {128, 128, 2, 4.0f, 1.10f}, {256, 256, 1, 5.0f, 1.36f}};
+  static const Shape shapes[] = {{32, 32, 1, 2.2f, 0.165f, 0.0f},  {64, 64, 1, 2.1f, 0.30f, 0.0f},
+                                 {64, 128, 1, 2.2f, 0.40f, 0.0f},  {128, 128, 1, 3.3f, 0.54f, 0.0f},
+                                 {128, 192, 1, 5.2f, 0.62f, 0.0f}, {128, 128, 2, 4.0f, 1.10f, 0.0f},
+                                 {256, 256, 1, 1.3f, 1.30f, 6.5f}};
   constexpr int TILE = 5, BIG = 6;
   const int cus = kg_cu_count();
-  // the persistent kernel's epilogue stores 16-byte chunks of 8 columns, and below 256 tiles it is never the best
-  const bool big_ok = (long long)((m + 255) / 256) * ((n + 255) / 256) >= 256 && n % 8 == 0 && ldc % 8 == 0 &&
-                      kg_aligned(c, 16) && (long long)rows * ldc * 2 < (1ll << 31);
-  if (big_ok) KG_CHECK((long long)rows * lda < (1ll << 31));
+  // the persistent kernel's epilogue stores 16-byte chunks of 8 columns, its offsets are 32-bit; calls of 256 of its
+  // tiles or more it could store need rows of A within its reach
+  const bool reach = (long long)rows * lda < (1ll << 31);
+  const bool stores = n % 8 == 0 && ldc % 8 == 0 && kg_aligned(c, 16) && (long long)rows * ldc * 2 < (1ll << 31);
+  if (stores && (long long)((m + 255) / 256) * ((n + 255) / 256) >= 256) KG_CHECK(reach);
+  const bool big_ok = stores && reach;
   int best = TILE;
   float best_t = 0.0f;
   long long tiles = 0;
   for (int i = 0; i <= (big_ok ? BIG : TILE); ++i) {
     const Shape& s = shapes[i];
     const long long t = ((m + s.bm - 1ll) / s.bm) * ((n + s.bn - 1ll) / s.bn), slots = (long long)s.per_cu * cus;
-    const float us = (float)((t + slots - 1) / slots) * (s.fixed + s.block * (float)(k >> 7));
+    const float us = s.start + (float)((t + slots - 1) / slots) * (s.fixed + s.block * (float)(k >> 7));
     if (i == 0 || us < best_t) best = i, best_t = us, tiles = t;
   }
   KG_CHECK(tiles < (1ll << 31));

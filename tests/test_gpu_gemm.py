@@ -134,6 +134,26 @@ def test_fp8_gemm_tile_shapes(M, N, K):
     assert np.all(out[:M, N:] == SENTINEL) and np.all(out[M:] == SENTINEL)
 
 
+@pytest.mark.parametrize("M,N,K", [(4200, 4096, 1024), (5000, 2752, 6144), (2300, 6144, 16384), (11000, 1024, 512)])
+def test_fp8_gemm_pick_time(M, N, K):
+    """Dense GEMMs that 256 x 256 tiles cover in one round, or in two where the smaller tiles need three, are no slower
+    than the grouped entry point's 256 x 256 tiles over the same rows as one expert (they took 1.25 to 1.5 times it), and
+    equal it."""
+    g = synth.generator(M + N, "cuda")
+    rows = (M + 127) // 128 * 128
+    codes = lambda *s: torch.randint(0, 0x78, s, generator=g, device=DEV, dtype=torch.uint8)
+    sf = lambda r: torch.randint(118, 127, (ref.sf_words(K) * r * 4,), generator=g, device=DEV, dtype=torch.uint8)
+    a, w, sfa, sfb = codes(rows, K), codes(N, K), sf(rows), sf(N)
+    psum = torch.tensor([M], dtype=torch.int32, device=DEV)
+    c0, c1 = filled((rows, N), SENTINEL, torch.int16), filled((rows, N), SENTINEL, torch.int16)
+    dense, grouped = fastest([lambda: ops.fp8_gemm(a, w, sfa, sfb, c0, M, n=N, k=K, rows=rows, lda=K, ldc=N, sfa_rows=rows),
+                              lambda: ops.fp8_gemm_psum(a, w, sfa, sfb, c1, psum, n=N, k=K, rows=rows, lda=K, ldc=N,
+                                                        sfa_rows=rows, groups=1)])
+    print(f"dense {M}x{N}x{K}: {dense:.1f} us, as one group {grouped:.1f}", flush=True)
+    assert torch.equal(c0, c1)
+    assert dense <= 1.15 * grouped
+
+
 @pytest.mark.parametrize("N,K,ldc", [(2624, 6144, 2752), (16384, 2048, 20480), (6144, 16384, 6144)])
 def test_fp8_gemm_bench_shapes_sampled(N, K, ldc):
     """The bench's dense GEMMs at full size (M = 16384: q_a/kv_a, q_b, o_proj): activations quantized on the
