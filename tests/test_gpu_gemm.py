@@ -76,18 +76,28 @@ def model_on_rows(a, w, sfa, sfb, M, N, K, lda, sfa_rows, rows):
 
 # ------------------------------------------------------------------ dense (a2)
 
+# the persistent 256 x 256 kernel with row tails of 1-128 (half tiles) and 129-255 rows, column tails, and more K blocks
+# than one scale word holds (the picks are checked in test_dispatch.py)
+PERSISTENT = [
+    (4100, 3080, 1152, 4224, 1152, 3088, 4224),     # a row tail of 4, a column tail of 8, 9 K blocks
+    (1900, 6152, 896, 1900, 912, 6160, 1910),       # a row tail of 108, 7 K blocks, lda > k
+    (4000, 2632, 1536, 4096, 1536, 2632, 4096),     # a row tail of 160, 12 K blocks
+    (2300, 4168, 640, 2304, 640, 4176, 2300 + 8),   # a row tail of 252, 5 K blocks
+    (4000, 4160, 640, 4096, 640, 4224, 4096),
+    (4352, 4224, 896, 4352, 896, 4232, 4352),       # 17 x 17 tiles, a column tail of 128
+]
+
+
 @pytest.mark.parametrize("M,N,K,rows,lda,ldc,sfa_rows", [
     (512, 2048, 6144, 512, 6144, 2048, 512),        # the parity configuration
     (300, 2624, 1024, 320, 1152, 2752, 384),        # N tail of 64 (2624 = 20.5 x 128), ldc > n, lda > k
     (4096, 4096, 512, 4096, 512, 4096, 4096),       # 256 x 256 tiles
-    (4000, 4160, 640, 4096, 640, 4224, 4096),       # 256 x 256 tiles, M and N tails, odd K-block count
-    (4100, 4096, 1536, 4224, 1536, 4096, 4224),     # an M tail of 4 rows (half tiles), K = 3 x 512
+    (4100, 4096, 1536, 4224, 1536, 4096, 4224),     # 128 x 192 tiles, an M tail of 4 rows, K = 3 x 512
     (4096, 4096, 128, 4096, 128, 4096, 4096),       # one K block: three padded stages of four
-    (4352, 4224, 896, 4352, 896, 4232, 4352),       # 17 x 17 tiles, N tail of 128, ldc > n, K = 7 blocks
     (8192, 2048, 2560, 8192, 2560, 2048, 8192),     # K = 5 groups of four stages
-    (512, 256, 384, 512, 384, 256, 512),            # odd K-block count, 128 x 128 tiles
+    (512, 256, 384, 512, 384, 256, 512),            # odd K-block count, 32 x 32 tiles
     (1, 2048, 6144, 16, 6144, 2048, 16),            # a single row
-])
+] + PERSISTENT)
 def test_fp8_gemm(M, N, K, rows, lda, ldc, sfa_rows):
     a, sfa = quant_act(M, K, rows, lda, sfa_rows, seed=M + N + K)
     w, sfb = quant_weight(N, K, seed=N * 7 + K)
@@ -104,17 +114,21 @@ def test_fp8_gemm(M, N, K, rows, lda, ldc, sfa_rows):
     assert np.all(out[:M, N:] == SENTINEL) and np.all(out[M:] == SENTINEL)
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (1, 5, 128), (31, 100, 640), (33, 97, 2176),       # 32 x 32 tiles: one K block, odd block counts, past a ring
-    (200, 1201, 384), (193, 1216, 1152),               # 64 x 64
-    (640, 1700, 128), (577, 1729, 1408),               # 64 x 128
-    (1000, 2500, 384), (897, 2433, 640),               # 128 x 128
-    (1500, 3300, 384), (1409, 3265, 1664),             # 128 x 192: fewer K blocks than stages, past a loop body
-    (2000, 3700, 256),                                 # two 128 x 128 workgroups per CU
-])
+# (rows, columns, workgroups a CU) of the tile -> sizes that the dense GEMM runs in it, with C rows of an odd stride
+TILE_SHAPES = {
+    (32, 32, 1): [(1, 5, 128), (31, 100, 640), (33, 97, 2176)],     # one K block, odd block counts, past a ring
+    (64, 64, 1): [(200, 1201, 384), (193, 1216, 1152)],
+    (64, 128, 1): [(640, 1700, 128), (577, 1729, 1408)],
+    (128, 128, 1): [(1000, 2500, 384), (897, 2433, 640)],
+    (128, 192, 1): [(1500, 3300, 384), (1409, 3265, 1664)],         # fewer K blocks than stages, past a loop body
+    (128, 128, 2): [(2000, 3700, 256)],
+}
+
+
+@pytest.mark.parametrize("M,N,K", [size for sizes in TILE_SHAPES.values() for size in sizes])
 def test_fp8_gemm_tile_shapes(M, N, K):
-    """Each tile shape the dense GEMM picks by size, with row, column and K remainders: sampled rows against the
-    oracle and its MFMA model at the bar of test_fp8_gemm, nothing written past m and n."""
+    """Each tile shape the dense GEMM picks by size (test_dispatch.py checks the picks), with row, column and K
+    remainders: sampled rows against the oracle and its MFMA model at the bar of test_fp8_gemm, nothing written past m and n."""
     print(f"fp8 gemm {M}x{N}x{K}", flush=True)
     ldc = (N + 3) // 4 * 4 + 4
     a, sfa = quant_act(M, K, M, K, M, seed=M + 5 * N + K)
@@ -440,8 +454,29 @@ def test_bf16_batched_contiguous_k128():
     bf16_ref_check(h(D, np.uint16), A, B, 128, "k128")
 
 
+# 64 heads and one head over the 256-column tiles of the batched kernel, with row and column tails
+WIDE_BATCHED = [(64, 513, 264, 128)]
+WIDE_F32 = [(33000, 264, 64, 272)]
+
+
+@pytest.mark.parametrize("heads,m,n,k", WIDE_BATCHED)
+def test_bf16_batched_wide_tiles_tail(heads, m, n, k):
+    """Enough 128 x 256 tiles for the batched kernel to take them, their last column tile partial: against the oracle,
+    nothing written past m and n."""
+    print(f"bf16 batched {heads} heads {m} x {n} x {k}", flush=True)
+    g = synth.generator(heads + m)
+    A = torch.randn(m + 2, heads, k, generator=g).to(torch.bfloat16)
+    B = (torch.randn(heads, n, k, generator=g) * 0.05).to(torch.bfloat16)
+    D = filled((m + 2, heads, n + 8), SENTINEL, torch.int16)
+    ops.bf16_batched(A.to(DEV), B.to(DEV), D, m, n=n, k=k, rows=m + 2, a_strides=(heads * k * 2, k * 2),
+                     b_strides=(k * 2, n * k * 2), d_strides=(heads * (n + 8) * 2, (n + 8) * 2), heads=heads)
+    out = h(D, np.uint16)
+    bf16_ref_check(np.ascontiguousarray(out[:m, :, :n]), A[:m], B, k, f"wide {heads}x{m}x{n}x{k}")
+    assert np.all(out[:m, :, n:] == SENTINEL) and np.all(out[m:] == SENTINEL)
+
+
 @pytest.mark.parametrize("m,n,k,ldc", [(1000, 256, 6144, 256), (333, 32, 6144, 40), (16, 264, 192, 272),
-                                       (40000, 256, 128, 256)])
+                                       (40000, 256, 128, 256)] + WIDE_F32)
 def test_gemm_f32_and_bf16(m, n, k, ldc):
     """The manifest's library GEMMs (scripts/gen.py:99-102): the MoE router's f32-output one (gen.py:435) and the
     indexer's bf16 weights_proj (gen.py:368), C = A . B^T; columns past n of each ldc row untouched."""
@@ -465,12 +500,16 @@ def test_gemm_f32_and_bf16(m, n, k, ldc):
     assert ok, ref.parity_line(f"gemm_bf16 {m}x{n}x{k}", rep)
 
 
+# the 128 x 128 ring of the wide long-K library GEMMs: the bench's shape, and with row and column tails and an odd K
+LIBRARY_128 = [(16384, 256, 6144, 256), (16001, 264, 1088, 272)]
+
+
 @pytest.mark.parametrize("m,n,k,ldc", [(1000, 256, 6144, 264), (333, 32, 6144, 40), (130, 24, 1024, 24),
-                                       (257, 72, 2048, 80), (64, 200, 1088, 208), (16384, 256, 6144, 256),
-                                       (16384, 32, 6144, 32), (100, 64, 1216, 72), (77, 48, 3136, 56)])
+                                       (257, 72, 2048, 80), (64, 200, 1088, 208), (16384, 32, 6144, 32),
+                                       (100, 64, 1216, 72), (77, 48, 3136, 56)] + LIBRARY_128)
 def test_gemm_long_k_matches_batched(m, n, k, ldc):
-    """Library GEMMs with K >= 1024 run the long-K kernels.  For n > 64 (the multi-stage ring) the sums are the
-    batched kernel's bit for bit (same MFMA chain over K; one head of kg_bf16_batched is the comparison); for
+    """Library GEMMs with K >= 1024 run the long-K kernels.  For n > 64 (rings of several stages, in 32 x 32, 64 x 64 or
+    128 x 128 tiles by size) the bf16 outputs are the batched kernel's bit for bit (same MFMA chain over K; one head of kg_bf16_batched is the comparison); for
     n <= 64 (four K quarters summed in wave order) they are within the fp32 reference's accumulation bound.  bf16
     and f32 out, with row / column tails and columns past n of each ldc row untouched, and the f32 sums rounding
     to exactly the bf16 outputs (one set of sums, one rounding)."""
@@ -503,10 +542,14 @@ def test_gemm_long_k_matches_batched(m, n, k, ldc):
     assert np.array_equal(rb, D[:, :n])
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 72, 1024), (33, 264, 1088), (1300, 200, 1088), (2100, 264, 1984)])
+LIBRARY_FEW = [(1, 72, 1024), (33, 264, 1088), (1300, 200, 1088), (2100, 264, 1984)]
+
+
+@pytest.mark.parametrize("m,n,k", LIBRARY_FEW)
 def test_gemm_few_rows_matches_batched(m, n, k):
     """The wide library GEMMs of few rows, in 32 x 32 and 64 x 64 tiles (by size) with row and column remainders and
-    odd counts of 64-wide K steps: the batched kernel's f32 sums bit for bit, and the bf16 outputs their rounding."""
+    odd counts of 64-wide K steps: the bf16 outputs, and the f32 outputs rounded to bf16, are the batched kernel's bit
+    for bit, and the f32 outputs are within the accumulation bound of the exact sums."""
     g = synth.generator(11 * m + n)
     A = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
     B = (torch.randn(n, k, generator=g) * 0.02).to(torch.bfloat16).to(DEV)

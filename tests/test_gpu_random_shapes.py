@@ -1,6 +1,6 @@
 """Seeded random shapes through the GEMMs and the prefill top-k, beyond the hand-picked edge cases: dense fp8
-GEMMs on both kernels (the 128 x 128 tile kernel for small or odd-width outputs, the persistent one for at
-least 256 tiles of 256 x 256) with random tails, strides and scale-row counts; grouped GEMMs with random
+GEMMs (tiles of 32 x 32 to 128 x 128 for the small or odd-width outputs, the persistent 256 x 256 kernel for the
+large ones) with random tails, strides and scale-row counts; grouped GEMMs with random
 expert counts; top-k rows of random lengths, starts and K.  Each case against the oracle, at the same bars
 as the fixed cases (fp8 GEMMs: rel-L2 against the fp32 reference and equality with the oracle's model of
 the fp8 MFMA on sampled rows; top-k bit for bit)."""
@@ -127,9 +127,9 @@ def test_quant_and_silu_random(seed):
 
 @pytest.mark.parametrize("seed", [1, 2, 3, 6])
 def test_bf16_batched_random(seed):
-    """The head-batched bf16 GEMM at random heads, rows, widths and K, with padded row / head strides (n below
-    256 takes 128-column tiles, from 256 on 256-column ones: seeds 3 and 6 give n = 400 and 264, a partial
-    last column tile)."""
+    """The head-batched bf16 GEMM at random heads, rows, widths and K, with padded row / head strides, in 128-column
+    tiles (these sizes have too few 256-column ones; seeds 3 and 6 give n = 400 and 264, a partial last column
+    tile)."""
     from kern_glm53_amd import synth
     from tests.test_gpu_gemm import bf16_ref_check
     rng = np.random.default_rng(500 + seed)
