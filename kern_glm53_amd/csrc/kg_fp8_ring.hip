@@ -6,9 +6,9 @@
 // identical), K is never split, and the only parallelism is over output tiles.  With a ring of two stages a workgroup
 // waits for a memory round trip per K block (0.9 us of a 128 x 128 x 128 block whose MFMAs take 0.2); here NS stages
 // are in flight, and the tile shapes below let a GEMM of any size spread over the CUs in about one round.  What is
-// left per block is the copy into LDS: a CU takes 97-105 GB/s of operands that sit in its L2 and 62 GB/s while they
-// come from HBM, whatever the ring's depth, the number of waves or the path (VGPRs or LDS), so a block of 128 x 192
-// (40 KB) takes 0.68 us where its MFMAs take 0.32.  Weights from HBM, M x N x K, two-stage ring -> this one: 7 x 2752
+// left per block is the copy into LDS: a CU takes 86-103 GB/s of operands that sit in its L2 (tiles of 64 x 64 on) and
+// 62-67 GB/s in a GEMM whose weights come from HBM, whatever the ring's depth, the number of waves or the path (VGPRs or
+// LDS), so a block of 128 x 192 (40 KB) takes 0.61-0.68 us where its MFMAs take 0.32.  Weights from HBM, M x N x K, two-stage ring -> this one: 7 x 2752
 // x 6144 43 -> 10.7 us, 150 x 20480 x 2048 25 -> 18, 420 x 6144 x 12288 88 -> 62, 1000 x 6144 x 16384 147 -> 97.
 //
 // Kernel.  NW waves, of which WM x WN compute: wave (wm, wn) owns TJ x TI MFMA tiles of 32 x 32 (v_mfma_scale

@@ -9,13 +9,14 @@
 // column tile (256 weight rows) of one expert and half the registers, so that two share a CU: one streams while the
 // other starts or ends, and they keep 100 to 200 KB in flight.
 //   * A wave owns 64 weight rows (modes 1: 64 columns; 2: 32 gate rows and their 32 up rows) over all the expert's
-//     rows.  Weight fragments go from HBM into registers, D stages of 128 K ahead; activations through a ring of D + 2
-//     LDS stages, D ahead as well (the workgroup's four waves share them).
+//     rows.  Weight fragments go from HBM into registers, D stages of 128 K ahead; activations through a ring of NB = 4
+//     LDS stages, DA stages ahead (the workgroup's four waves share them).
 //   * The weights are loaded non-temporally: each byte is used once (gate_up of 64 tokens 852 us without, 779 with).
-//   * Up to 64 rows: 2 MFMA tiles of 32 rows a wave, D = 4.  Up to 128: 4 tiles, D = 2.  Rows past the expert's
-//     end are not loaded (zeros).
-//   * One barrier a stage: this wave's copies of the next stage have landed (the loads issued after them are D - 1
-//     stages' weights and copies, and loads complete in issue order) and its reads of this stage are done.
+//   * Up to 64 rows: 2 MFMA tiles of 32 rows a wave, D = 4, DA = 3.  Up to 128: 4 tiles, D = DA = 2.  Rows past the
+//     expert's end are not loaded (zeros).
+//   * One barrier a stage: this wave's copies of the next stage have landed (issued DA stages before it; since then that
+//     stage's weights and DA - 1 stages' copies and weights, and loads complete in issue order) and its reads of this
+//     stage are done.
 //   * A stage past K (the scale words hold four) multiplies zeros, as in the persistent kernel, so that even the sign
 //     of a zero agrees.
 #include "kg_fp8_common.h"
@@ -145,7 +146,7 @@ __global__ __launch_bounds__(256, 2) void kg_fp8_gemm_wfew(const KgFp8Args p) {
         wb[x][o] = __builtin_amdgcn_raw_buffer_load_b32(rsb, (unsigned)((wr[o] + (lane & 31)) * 4 + kg * p.n * 4), 0, 0);
     };
     auto stage = [&](auto ss, int s) __attribute__((always_inline)) {
-      constexpr int S = decltype(ss)::value;                              // s % 8: ring slot, weight set, scale byte
+      constexpr int S = decltype(ss)::value;                              // s % 4: ring slot, weight set, scale byte
       constexpr int PH = S & 3, G = 0;
       if constexpr (PH == 0) {
         const int live = KB - s;
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(256, 2) void kg_fp8_gemm_wfew(const KgFp8Args p) {
       __builtin_amdgcn_sched_barrier(0);
       wload(S % D, s + D);
       __builtin_amdgcn_sched_barrier(0);
-      // the copies of stage s + 1 were issued in stage s + 1 - D: since then that stage's weights and D - 1 stages'
+      // the copies of stage s + 1 were issued in stage s + 1 - DA: since then that stage's weights and DA - 1 stages'
       // copies and weights (the scale words only add)
       kg_ring_barrier<YOUNGER>();
       __builtin_amdgcn_sched_barrier(0);

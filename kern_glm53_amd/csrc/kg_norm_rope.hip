@@ -1,8 +1,9 @@
 // The operand producers upstream of the glm_deepgemm GEMMs, rebuilt for gfx950: residual add + RMSNorm +
 // activation quant (glm_add_rms_quant, source/glm_glue.cu:127-162), the MLA projection's norms, rope and
 // cache writes (glm_mla_prep / glm_mla_prep_fp8, 196-299) and the query post-processing after q_b
-// (glm_q_post, 301-351).  HBM-bound row work: one wave64 per row, four rows per 256-thread workgroup,
-// 16-byte accesses, every reduction inside the wave (no LDS, no barrier).
+// (glm_q_post, 301-351).  HBM-bound row work: one wave64 per row for the residual norm, two for the MLA projection, two or
+// four for the query, four waves per 256-thread workgroup, 16-byte accesses, every reduction inside a wave (no LDS, no
+// barrier).
 //
 // Numerics follow the reference bit for bit except where it calls CUDA's approximate rsqrtf, which
 // becomes the correctly rounded 1 / sqrt (HIP's sqrtf and '/' are IEEE-rounded by default).  The sums of

@@ -11,12 +11,14 @@ normed row to the block's output h, with the gate_up GEMM and `silu_moe` fused i
             (the weights in fragment order, derived at load time)     kg_fp8_gemm_psum without them)
     shared  gate_up with the SiLU-mul-quant epilogue (one group: rows   (kg_fp8_gemm_psum_silu_quant,
             [0, T)), down on xq -> sh                                    kg_fp8_gemm)
-            (a chunk of x_rows not a multiple of 128: the dense gate_up  (kg_fp8_gemm, kg_silu_mul_quant)
-            GEMM into bf16, then silu_mul_quant, as the reference does)
+            (calls of at most SHARED_PAIR_ROWS tokens, or x_rows not a   (kg_fp8_gemm, kg_silu_mul_quant)
+            multiple of 128: the dense gate_up GEMM into bf16, then
+            silu_mul_quant, as the reference does; the same outputs)
     combine h = bf16(sh + sum_k wts f2)                                 (kg_moe_combine)
 
 Buffers follow the reference's sizes (scripts/gen.py:86-87, 285-300): mcap = 8 T + 256 * 128 routed-row slots,
-scale words for `x_rows` rows (the chunk).  Every buffer is allocated once by `MoEBuffers`; a call allocates
+scale words for `x_rows` rows (the chunk), and for the shared expert's bf16 gate_up up to 16 MB (x_rows rows where those
+are not a multiple of 128).  Every buffer is allocated once by `MoEBuffers`; a call allocates
 nothing, and with T = MoEBuffers.T (the default) every launch of the block is one of this library's kernels.  The routed-row buffers start zeroed: the GEMMs read (and never store) their padding rows.  Weights
 are the reference's operand layouts (glm_requant's output): w13 [256 * 4096][6144] with scale words
 [256 * 12][4096], w2 [256 * 6144][2048] with [256 * 4][6144], the shared expert's w_sgu [4096][6144] /

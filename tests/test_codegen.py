@@ -24,7 +24,7 @@ def _asm(tmp_path, source="kg_fp8_gemm.hip"):
     except RuntimeError:
         pytest.skip("hipcc not available")
     out = tmp_path / (pathlib.Path(source).stem + ".s")
-    flags = [f for f in build.COMMON if f != "-fPIC"]
+    flags = [f for f in build.COMMON if f != "-fPIC"] + build.SOURCES[source]
     cmd = [cc, *flags, "--cuda-device-only", "-S", str(build.CSRC / source), "-o", str(out)]
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
@@ -79,3 +79,43 @@ def test_batched_gemm_fits_its_occupancy(tmp_path):
             assert m["vgpr_count"] + m["agpr_count"] <= regs, (name, m)
             assert m["vgpr_spill_count"] == 0 and m["sgpr_spill_count"] == 0, (name, m)
             assert m["group_segment_fixed_size"] == lds, (name, m)
+
+
+def _regs(m):
+    """Registers a lane of the 512 a SIMD lane has (the total: AGPRs follow the VGPRs)."""
+    return m["vgpr_count"]
+
+
+def test_ring_gemms_fit_and_do_not_spill(tmp_path):
+    """The deep-ring kernels take most of a CU's LDS and wait by counting loads: a spill's reload would be one more.  One
+    wave a SIMD may use all 512 registers, the 128 x 128 tile's eight waves (two a SIMD) 256."""
+    meta = _kernel_meta(_asm(tmp_path, "kg_fp8_ring.hip"))
+    ring = {n: m for n, m in meta.items() if "kg_fp8_gemm_ring" in n}
+    assert len(ring) == 5, sorted(meta)
+    for name, m in ring.items():
+        assert m["vgpr_spill_count"] == 0 and m["sgpr_spill_count"] == 0, (name, m)
+        assert _regs(m) <= (256 if "ILi4ELi2E" in name else 512), (name, m)
+        assert m["group_segment_fixed_size"] <= 160 * 1024, (name, m)
+
+
+def test_few_row_kernels_fit_and_do_not_spill(tmp_path):
+    """kg_fp8_gemm_wfew shares a CU between two workgroups (at most 256 registers a lane, 80 KB of LDS each); the few-row
+    library GEMM counts its loads like the rings."""
+    meta = _kernel_meta(_asm(tmp_path, "kg_fp8_wfew.hip"))
+    for mode in (1, 2):
+        m = meta[f"_Z16kg_fp8_gemm_wfewILi{mode}EEv9KgFp8Args"]
+        assert _regs(m) <= 256 and m["group_segment_fixed_size"] <= 80 * 1024, (mode, m)
+        assert m["vgpr_spill_count"] == 0 and m["sgpr_spill_count"] == 0, (mode, m)
+    few = {n: m for n, m in _kernel_meta(_asm(tmp_path, "kg_bf16_batched.hip")).items() if "kg_gemm_few_kernel" in n}
+    assert len(few) == 4
+    for name, m in few.items():
+        assert m["vgpr_spill_count"] == 0 and m["sgpr_spill_count"] == 0, (name, m)
+
+
+def test_mqa_logits_fits_two_workgroups(tmp_path):
+    """Eight waves a workgroup, two workgroups a CU: at most 128 registers a lane and 80 KB of LDS.  No hidden kernel
+    arguments (gridDim): they cost a launch of a few rows 0.45 us."""
+    m = _kernel_meta(_asm(tmp_path, "kg_mqa_logits.hip"))["_Z20kg_mqa_logits_kernelPKhS0_PKfS2_PKjS4_Pfiiiii"]
+    assert _regs(m) <= 128 and m["group_segment_fixed_size"] <= 80 * 1024, m
+    assert m["vgpr_spill_count"] == 0 and m["sgpr_spill_count"] == 0, m
+    assert m["kernarg_segment_size"] < 256, m
